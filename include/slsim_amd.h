@@ -227,8 +227,10 @@ typedef struct {
  * (FullRange/internal_rayshooter_multi.cpp:53-251; include/lens.h:913-1103).
  * Host buffers: x (2n, x0 x1 interleaved, radians), zs (n source redshifts or
  * NULL = lens source), y (2n out), A (4n out, row-major a0 a1 a2 a3).
- * Rays are Morton-ordered on the device so that each wavefront walks a
- * spatially coherent bundle; results come back in input order.
+ * Large lists are Morton-ordered on the device so that each wavefront walks a
+ * spatially coherent bundle; short lists take a wavefront or more per ray, in
+ * FP64 (SLSIM_FP32C too: nothing is then left to guard, n_guarded is 0).
+ * Results come back in input order.
  */
 int slsim_shoot(slsim_lens lens, size_t n, const double* x, const double* zs, double* y,
                 double* A, int precision, slsim_shoot_stats* stats);

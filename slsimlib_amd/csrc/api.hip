@@ -822,6 +822,20 @@ void make_steps_into(const slsim_lens_s* L, const RayState& st, int64_t nslots,
   }
 }
 
+// Every plane of particle trees only (trees uploaded).
+static bool particle_planes(const slsim_lens_s* L) {
+  for (int h : L->tree_hcnt)
+    if (h > 0) return false;
+  return true;
+}
+
+// Whether a list of n rays goes to the lone-ray FP64 walk (either precision:
+// its FP64 results need no guard).
+bool list_is_lone(const slsim_lens_s* L, size_t n, int precision) {
+  if (precision != SLSIM_FP64 && precision != SLSIM_FP32C) return false;
+  return n <= (precision == SLSIM_FP64 ? kLoneRays64 : kLoneRays32) && particle_planes(L);
+}
+
 void make_steps(const slsim_lens_s* L, const RayState& st, int64_t nslots, uint32_t* counters,
                 std::vector<StepJob>& steps) {
   steps.resize(L->plane_redshifts.size() - 1);
@@ -833,6 +847,8 @@ void make_steps(const slsim_lens_s* L, const RayState& st, int64_t nslots, uint3
 namespace {
 
 // Runs the plane steps [0, jmax) of one job on the context stream.
+// lone_rays > 0: rays 0 .. lone_rays - 1 by the lone-ray walk; then nothing
+// waits for the steps unless they are timed.
 int run_steps(slsim_ctx c, const StepJob* djobs, const StepJob* steps, int jmax,
               uint32_t nbundles, int precision, bool count, uint32_t* err,
               slsim_shoot_stats* stats, uint32_t lone_rays = 0) {
@@ -843,13 +859,14 @@ int run_steps(slsim_ctx c, const StepJob* djobs, const StepJob* steps, int jmax,
   for (int j = 0; j < jmax; ++j) {
     if (timed) SLSIM_HIP_CHECK(hipEventRecord(ev[2 * j], c->stream));
     if (lone_rays > 0)
-      launch_plane_step_lone(c->stream, djobs + j, lone_rays, err);
+      launch_plane_step_lone(c->stream, lone_waves(lone_rays), djobs + j, nullptr, lone_rays);
     else
       launch_plane_step(precision, count, nbundles, c->stream, djobs + j, nullptr, err,
                         steps[j].nhtrees > 0 ? steps[j].hkind : 0);
     if (timed) SLSIM_HIP_CHECK(hipEventRecord(ev[2 * j + 1], c->stream));
   }
   SLSIM_HIP_CHECK(hipGetLastError());
+  if (lone_rays > 0 && !timed) return SLSIM_OK;
   SLSIM_HIP_CHECK(hipStreamSynchronize(c->stream));
   if (timed) {
     double tot = 0, mx = 0;
@@ -883,45 +900,10 @@ int guard_refine(slsim_lens L, const RayState& st, int64_t nslots, const GuardMa
                  int64_t nrays, const double* zs_dev, double zs_uniform, double* y_dev,
                  double* A_dev, ScratchT& s, int32_t* nguard);
 
-// rayshooterInternal on device buffers (FullRange/internal_rayshooter_multi.cpp:
-// 53-251): rays Morton-ordered into 64-ray bundles, one launch per plane, the
-// results scattered back to input order.  Device scratch comes from `s`
-// (the context's cache, or the fixed array of the no-allocation entry
-// point); the lens's trees must be resident.  Host buffers are fixed-size
-// arrays, so a call allocates nothing beyond `s`.
+// The Morton order of the rays, so that each wavefront gets a compact bundle.
 template <typename ScratchT>
-int shoot_array(slsim_lens L, size_t n, const double* x_dev, const double* zs_dev,
-                double* y_dev, double* A_dev, int precision, slsim_shoot_stats* stats,
-                ScratchT& s, int lanes = kWave, double zs_uniform = 0.0) {
-  const double t0 = now_ms();
-  if (precision < SLSIM_FP64 || precision > SLSIM_DIRECT64) return arg_error("bad precision");
-  if (stats) std::memset(stats, 0, sizeof(*stats));
-  if (n == 0) return SLSIM_OK;
-  if (!x_dev || !y_dev || !A_dev) return arg_error("null buffer");
-  if (n >= (size_t)1 << 32) return arg_error("too many rays in one call");
-  if (L->trees_dirty) return arg_error("lens trees are not on the device");
-  slsim_ctx c = L->ctx;
-  const int nplanes = (int)L->plane_redshifts.size() - 1;
-  if (nplanes > kMaxPlanesFixed && !ScratchT::kMayAllocate)
-    return arg_error("too many lens planes for the no-allocation entry point");
-  // lanes == 0: one wavefront per ray (the lone-ray FP64 walk) where every
-  // plane has particle trees only, else full bundles; rays dense in the state
-  const bool lone_asked = lanes == 0;
-  if (lone_asked) lanes = kWave;
-  if (lanes < 1 || lanes > kWave) return arg_error("bad rays per bundle");
-  const int64_t nbundles = ((int64_t)n + lanes - 1) / lanes;
-  const int64_t nslots = nbundles * kWave;
+int morton_order(slsim_ctx c, int64_t n, const double* x_dev, ScratchT& s, uint32_t** out) {
   int rc;
-  RayState st;
-  {
-    char* d;
-    if ((rc = s.get(&d, kStateBytesPerSlot * (size_t)nslots))) return rc;
-    st = state_view(reinterpret_cast<double*>(d), nslots);
-  }
-  uint32_t* err;
-  if ((rc = s.get(&err, 1))) return rc;
-  launch_zero_u32(c->stream, err, 1);
-  // Morton order of the rays: each wavefront gets a compact bundle
   const int nblk = (int)std::min<int64_t>(kMinmaxBlocks, (n + 255) / 256);
   double* part;
   if ((rc = s.get(&part, 4 * (size_t)nblk))) return rc;
@@ -948,29 +930,79 @@ int shoot_array(slsim_lens L, size_t n, const double* x_dev, const double* zs_de
   if ((rc = s.get(&stmp, sb))) return rc;
   SLSIM_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(stmp, sb, code, code_s, idx, perm, (int)n, 0,
                                                      30, c->stream));
+  *out = perm;
+  return SLSIM_OK;
+}
+
+// rayshooterInternal on device buffers (FullRange/internal_rayshooter_multi.cpp:
+// 53-251): rays Morton-ordered into 64-ray bundles, one launch per plane, the
+// results scattered back to input order.  Device scratch comes from `s`
+// (the context's cache, or the fixed array of the no-allocation entry
+// point); the lens's trees must be resident.  Host buffers are fixed-size
+// arrays, so a call allocates nothing beyond `s`.
+template <typename ScratchT>
+int shoot_array(slsim_lens L, size_t n, const double* x_dev, const double* zs_dev,
+                double* y_dev, double* A_dev, int precision, slsim_shoot_stats* stats,
+                ScratchT& s, int lanes = -1, double zs_uniform = 0.0) {
+  const double t0 = now_ms();
+  if (precision < SLSIM_FP64 || precision > SLSIM_DIRECT64) return arg_error("bad precision");
+  if (stats) std::memset(stats, 0, sizeof(*stats));
+  if (n == 0) return SLSIM_OK;
+  if (!x_dev || !y_dev || !A_dev) return arg_error("null buffer");
+  if (n >= (size_t)1 << 32) return arg_error("too many rays in one call");
+  if (L->trees_dirty) return arg_error("lens trees are not on the device");
+  slsim_ctx c = L->ctx;
+  const int nplanes = (int)L->plane_redshifts.size() - 1;
+  if (nplanes > kMaxPlanesFixed && !ScratchT::kMayAllocate)
+    return arg_error("too many lens planes for the no-allocation entry point");
+  // lanes < 0: the list's own rule; 0: the lone-ray FP64 walk where every
+  // plane has particle trees only, else full bundles.  Lone rays are dense in
+  // the state, in the list's order.
+  const bool guard_after = precision == SLSIM_FP32C && lanes < 0 && !list_is_lone(L, n, precision);
+  const bool lone = lanes == 0 ? precision == SLSIM_FP64 && particle_planes(L)
+                               : lanes < 0 && list_is_lone(L, n, precision);
+  if (lone) precision = SLSIM_FP64;
+  if (lanes <= 0) lanes = kWave;
+  if (lanes > kWave) return arg_error("bad rays per bundle");
+  const int64_t nbundles = ((int64_t)n + lanes - 1) / lanes;
+  const int64_t nslots = nbundles * kWave;
+  int rc;
+  RayState st;
+  {
+    char* d;
+    if ((rc = s.get(&d, kStateBytesPerSlot * (size_t)nslots))) return rc;
+    st = state_view(reinterpret_cast<double*>(d), nslots);
+  }
+  uint32_t *err = nullptr, *perm = nullptr;
+  if (!lone) {
+    if ((rc = s.get(&err, 1))) return rc;
+    launch_zero_u32(c->stream, err, 1);
+    if ((rc = morton_order(c, (int64_t)n, x_dev, s, &perm))) return rc;
+  }
   int32_t jmax = 0;
   double aal = 0, bbl = 0;
   if (nplanes > 0 && !zs_dev) uniform_source(L, zs_uniform, &jmax, &aal, &bbl);
-  double *zpl, *dl;
-  if ((rc = s.get(&zpl, L->plane_redshifts.size())) || (rc = s.get(&dl, L->Dl.size()))) return rc;
-  SLSIM_HIP_CHECK(hipMemcpyAsync(zpl, L->plane_redshifts.data(), 8 * L->plane_redshifts.size(),
-                                 hipMemcpyHostToDevice, c->stream));
-  SLSIM_HIP_CHECK(hipMemcpyAsync(dl, L->Dl.data(), 8 * L->Dl.size(), hipMemcpyHostToDevice, c->stream));
+  double *zpl = nullptr, *dl = nullptr;   // read for per-ray source redshifts only
+  if (zs_dev) {
+    if ((rc = s.get(&zpl, L->plane_redshifts.size())) || (rc = s.get(&dl, L->Dl.size()))) return rc;
+    SLSIM_HIP_CHECK(hipMemcpyAsync(zpl, L->plane_redshifts.data(), 8 * L->plane_redshifts.size(),
+                                   hipMemcpyHostToDevice, c->stream));
+    SLSIM_HIP_CHECK(hipMemcpyAsync(dl, L->Dl.data(), 8 * L->Dl.size(), hipMemcpyHostToDevice,
+                                   c->stream));
+  }
   FlatLCDM cosmo{L->Om, L->OL, L->h};
   launch_init_array(c->stream, st, nslots, (int64_t)n, perm, x_dev, nplanes > 0 ? zs_dev : nullptr,
                     jmax, aal, bbl, zpl, dl, nplanes, cosmo, lanes);
   const int steps_to_run = zs_dev ? nplanes : jmax;
+  StepJob steps_fixed[kMaxPlanesFixed];   // read by the copy until the stream is waited for
+  std::vector<StepJob> steps_more;
   if (steps_to_run > 0) {
-    StepJob steps_fixed[kMaxPlanesFixed];
-    std::vector<StepJob> steps_more;
     StepJob* steps = steps_fixed;
     if (nplanes > kMaxPlanesFixed) {
       steps_more.resize(nplanes);
       steps = steps_more.data();
     }
     make_steps_into(L, st, nslots, nullptr, steps);
-    bool lone = lone_asked && precision == SLSIM_FP64;
-    for (int j = 0; j < steps_to_run && lone; ++j) lone = steps[j].nhtrees == 0;
     StepJob* djobs;
     if ((rc = s.get(&djobs, (size_t)nplanes))) return rc;
     SLSIM_HIP_CHECK(hipMemcpyAsync(djobs, steps, sizeof(StepJob) * (size_t)nplanes,
@@ -981,8 +1013,9 @@ int shoot_array(slsim_lens L, size_t n, const double* x_dev, const double* zs_de
   }
   launch_finalize_array(c->stream, st, nslots, (int64_t)n, perm, y_dev, A_dev, lanes);
   SLSIM_HIP_CHECK(hipGetLastError());
-  if ((rc = check_err(c, err))) return rc;
-  if (precision == SLSIM_FP32C && steps_to_run > 0 && lanes == kWave && !lone_asked) {
+  if (lone) SLSIM_HIP_CHECK(hipStreamSynchronize(c->stream));
+  else if ((rc = check_err(c, err))) return rc;
+  if (guard_after && steps_to_run > 0) {
     GuardMap m{};
     m.perm = perm;
     m.x = x_dev;

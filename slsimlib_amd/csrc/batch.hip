@@ -525,6 +525,7 @@ struct slsim_server_s {
     int32_t jmax = 0, step = 0;
     int64_t nbundles = 0, next_bundle = 0;   // progress within plane `step`
     double aal = 0, bbl = 0;
+    bool lone = false;   // ray list on the lone-ray walk, as a call of its own would be
     std::vector<StepJob> steps;
     State state = PENDING;
     int status = SLSIM_OK;
@@ -576,6 +577,7 @@ int slsim_server_s::admit(Req* r) {
     slsim_lens_s* L = r->lens;
     if ((rc = L->upload_trees())) return rc;
     const int64_t n = r->nrays;
+    r->lone = list_is_lone(L, (size_t)n, r->precision);
     const int nplanes = (int)L->plane_redshifts.size() - 1;
     double* p = reinterpret_cast<double*>(base + ((sbytes + 255) & ~(size_t)255));
     r->xd = p;   p += 2 * n;
@@ -661,7 +663,7 @@ int slsim_server_s::iterate() {
     left -= t;
   }
   size_t nit = 0;
-  for (auto& t : take) nit += (size_t)t.second;
+  for (auto& t : take) nit += t.first->lone ? (size_t)t.first->nrays : (size_t)t.second;
   int rc = stage(take.size(), nit);
   if (rc) return rc;
   // jobs and items of all precisions in one staging copy, grouped by precision
@@ -672,7 +674,7 @@ int slsim_server_s::iterate() {
     item0[prec] = ni;
     for (auto& t : take) {
       Req* r = t.first;
-      if (r->precision != prec || t.second == 0) continue;
+      if (r->lone || r->precision != prec || t.second == 0) continue;
       h_jobs[nj] = r->steps[r->step];
       const uint32_t local = (uint32_t)(nj - job0[prec]);
       for (int64_t b = 0; b < t.second; ++b)
@@ -682,6 +684,25 @@ int slsim_server_s::iterate() {
   }
   job0[SLSIM_DIRECT64 + 1] = nj;
   item0[SLSIM_DIRECT64 + 1] = ni;
+  // lists on the lone-ray walk: a whole plane step each, grouped by the
+  // wavefronts their rays take
+  const int lone_w[2] = {1, 4};
+  size_t ljob0[3], litem0[3];
+  for (int g = 0; g < 2; ++g) {
+    ljob0[g] = nj;
+    litem0[g] = ni;
+    for (auto& t : take) {
+      Req* r = t.first;
+      if (!r->lone || t.second == 0 || lone_waves(r->nrays) != lone_w[g]) continue;
+      h_jobs[nj] = r->steps[r->step];
+      const uint32_t local = (uint32_t)(nj - ljob0[g]);
+      for (int64_t b = 0; b < r->nrays; ++b) h_items[ni++] = {local, (uint32_t)b};
+      ++nj;
+      t.second = r->nbundles - r->next_bundle;
+    }
+  }
+  ljob0[2] = nj;
+  litem0[2] = ni;
   SLSIM_HIP_CHECK(hipMemcpyAsync(d_jobs.p, h_jobs, sizeof(StepJob) * nj, hipMemcpyHostToDevice,
                                  stream));
   SLSIM_HIP_CHECK(hipMemcpyAsync(d_items.p, h_items, sizeof(WorkItem) * ni, hipMemcpyHostToDevice,
@@ -697,6 +718,10 @@ int slsim_server_s::iterate() {
                       static_cast<WorkItem*>(d_items.p) + item0[prec],
                       static_cast<uint32_t*>(d_err.p), halos);
   }
+  for (int g = 0; g < 2; ++g)
+    launch_plane_step_lone(stream, lone_w[g], static_cast<StepJob*>(d_jobs.p) + ljob0[g],
+                           static_cast<WorkItem*>(d_items.p) + litem0[g],
+                           (uint32_t)(litem0[g + 1] - litem0[g]));
   SLSIM_HIP_CHECK(hipGetLastError());
   // the staging buffers are reused next iteration
   SLSIM_HIP_CHECK(hipStreamSynchronize(stream));
@@ -766,7 +791,7 @@ void slsim_server_s::loop() {
       rc = SLSIM_ERR_TOO_DEEP;
     // the precision form's guard of each finished request, as a lone shoot's
     for (Req* r : finished) {
-      if (rc || r->precision != SLSIM_FP32C || r->jmax <= 0) continue;
+      if (rc || r->precision != SLSIM_FP32C || r->jmax <= 0 || r->lone) continue;
       GuardMap m{};
       if (r->nrays > 0) {
         m.x = r->xd;

@@ -1343,30 +1343,50 @@ void k_plane_step_nfw(const StepJob* __restrict__ jobs, const WorkItem* __restri
 }
 
 // ------------------------------------------------------- lone-ray FP64 walk
-// One plane step of one ray per wavefront, for a few scattered rays (the
-// precision form's guard), where a bundle walk would leave 63 lanes idle and
-// wait on one lane's stack: the lanes take the ray's cells 64 at a time from
-// an LDS stack (the last pushed first), a lane that opens an internal cell
-// pushes its children, and the particles of the opened leaves and of the big
-// lists the ray is near are then taken 64 at a time.  The cells, the opening
-// test and the terms are the FP64 walk's (include/quadTree.h:990-1128), so
-// the result is the bundle walk's up to the order of the FP64 sums; the
-// lanes' sums are added in a fixed order.
+// One plane step of one ray by NW wavefronts (one block), for lists of few or
+// scattered rays, where a bundle walk would leave lanes idle and wait on one
+// wavefront's serial traversal: the lanes take the ray's cells NW * 64 at a
+// time from an LDS stack (the last pushed first), a lane that opens an
+// internal cell pushes its children, and the particles of the opened leaves
+// and of the big lists the ray is near are listed in LDS and taken NW * 64 at
+// a time.  The cells, the opening test and the terms are the FP64 walk's
+// (include/quadTree.h:990-1128), so the result is the bundle walk's up to the
+// order of the FP64 sums, which is fixed by the ray and NW alone.
+//
+// What bounds it: the latency of a step (LDS stack, cell records from L2,
+// their far terms, the leaf particles' records), about 70 steps of 64 cells a
+// ray on a 2^20-particle plane, so few rays take more wavefronts each
+// (lone_waves) and the LDS is kept small for many rays in flight (10.3 KiB a
+// wavefront; with a 26 KiB stack and a binary search over the leaves for every
+// particle, 0.16 ms a plane of 500,000 particles for some hundred rays, now
+// 0.05).  A list of 40 rays of a 65,536-particle halo takes 0.13 ms (4.0 ms by
+// bundles), 3,001 rays through four planes of 200,000 0.92 ms (30 ms).  A pop takes
+// fewer cells as the stack fills, down to one (depth first, which grows by at
+// most 3 a level), so that the stack never overflows.
 namespace {
 
-// a pop of up to 64 cells pushes at most 256: 64 + 192 per level of depth
-constexpr int kLoneStack = 64 + 192 * 34;
+constexpr int kLoneStack = 1024;    // stack entries per wavefront of the block
+constexpr int kLoneItems = 1280;    // listed particles per wavefront (64 leaves of 20)
+constexpr int kLoneReserve = 3 * (kMaxLevels + 2) + 2;   // what depth-first growth can need
 
-__device__ inline int wave_prefix(int v, int& total) {
-  const int lane = lane_id();
-  int x = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
-  total = __shfl(x, 63, 64);
-  return x - v;
+// inclusive scan over the wavefront in registers (DPP row shifts and broadcasts)
+template <int CTRL, int ROWS>
+__device__ inline int dpp_or_zero(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+__device__ inline int wave_scan(int v) {
+  v += dpp_or_zero<0x111, 0xf>(v);   // row_shr:1
+  v += dpp_or_zero<0x112, 0xf>(v);   // row_shr:2
+  v += dpp_or_zero<0x114, 0xf>(v);   // row_shr:4
+  v += dpp_or_zero<0x118, 0xf>(v);   // row_shr:8
+  v += dpp_or_zero<0x142, 0xa>(v);   // row_bcast:15
+  v += dpp_or_zero<0x143, 0xc>(v);   // row_bcast:31
+  return v;
+}
+
+__device__ inline int lanes_before(uint64_t m) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                        __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
 __device__ inline double wave_sum(double v) {
@@ -1375,29 +1395,65 @@ __device__ inline double wave_sum(double v) {
   return v;
 }
 
-__device__ void lone_walk64(const TreeDesc& t, double rx, double ry, Acc64& a, int32_t* s_cell,
-                            int32_t* s_pst, int32_t* s_pcnt, int32_t* s_pkind, int32_t* s_pre,
-                            uint32_t* __restrict__ err) {
-  const int lane = lane_id();
+// a listed particle: a leaf's as a point mass, with its B-spline correction
+// when it is big and the leaf near (kind 1), or an internal cell's big
+// particle's correction (kind 2)
+__device__ __forceinline__ void lone_particle(const PartD& p, int kind, double rx, double ry,
+                                              double ia, Acc64& a) {
+  const double d0 = p.x - rx, d1 = p.y - ry;
+  double rr = d0 * d0 + d1 * d1;
+  if (rr < 1e-20) rr = 1e-20;
+  const double m = p.m;
+  if (kind != 2) {
+    const double inv = rcp64(rr);
+    const double pref = m * inv * kInvPI;
+    a.ax += (ia * m - pref) * d0;
+    a.ay += (ia * m - pref) * d1;
+    const double tmp = -2.0 * pref * inv;
+    a.g0 += 0.5 * (d0 * d0 - d1 * d1) * tmp;
+    a.g1 += d0 * d1 * tmp;
+    a.k -= m * ia;
+  }
+  if (kind == 2 || (kind == 1 && !signbit(p.h))) {
+    const double size = p.h;
+    if (rr < 4 * size * size) bspline64(d0, d1, sqrt(rr), m, size, a.ax, a.ay, a.k, a.g0, a.g1);
+  }
+}
+
+template <int NW>
+struct LoneShared {
+  int32_t cell[NW * kLoneStack];
+  uint32_t item[NW * kLoneItems];
+  uint8_t kind[NW * kLoneItems];
+  int32_t nch[NW], np[NW];
+  double sum[NW][5];
+};
+
+template <int NW>
+__device__ void lone_walk64(const TreeDesc& t, double rx, double ry, Acc64& a, LoneShared<NW>& s) {
+  const int tid = (int)threadIdx.x, w = uni(tid >> 6), lane = lane_id();
   const NodeD* __restrict__ nodes = t.nodesD;
   const PartD* __restrict__ parts = t.partsD;
   const PartD* __restrict__ bigs = t.bigD;
   const double ia = t.inv_area;
-  if (lane == 0) s_cell[0] = 0;
+  constexpr int kCap = NW * kLoneStack;
+  if (tid == 0) s.cell[0] = 0;
   int sp = 1;
   __syncthreads();
   while (sp > 0) {
-    const int c = sp < kWave ? sp : kWave;
+    // sp + 3 c <= kCap - kLoneReserve, or one cell at a time
+    const int room = (kCap - kLoneReserve - sp) / 3;
+    int c = sp < NW * kWave ? sp : NW * kWave;
+    if (c > room) c = room > 1 ? room : 1;
     sp -= c;
-    const int cell = lane < c ? s_cell[sp + lane] : -1;
-    __syncthreads();
-    int child = 0, cmask = 0, pst = 0, pcnt = 0, pkind = -1;
+    const int cell = tid < c ? s.cell[sp + tid] : -1;
+    int child = 0, cmask = 0, pst = 0, pcnt = 0, pkind = 0;
     if (cell >= 0) {
       const NodeD nd = nodes[cell];
       const double dx = nd.cx - rx, dy = nd.cy - ry;
       const double r2 = dx * dx + dy * dy;
       const bool nearc = r2 < nd.near2;
-      if (!(r2 < nd.r2crit || nearc)) {
+      if (!(r2 < nd.T)) {
         // far cell: monopole + quadrupole (include/quadTree.h:1089-1123)
         const double inv = rcp64(r2);
         const double mi = nd.mass * inv * kInvPI;
@@ -1421,109 +1477,122 @@ __device__ void lone_walk64(const TreeDesc& t, double rx, double ry, Acc64& a, i
       } else {
         child = nd.child;
         cmask = nd.cmask;
-        if (nd.count > 0 && nearc) {
+        if (nearc) {
           pst = nd.start;
           pcnt = nd.count;
           pkind = 2;
         }
       }
     }
-    // children onto the stack, in lane order
-    int nch_total = 0;
-    int at = sp + wave_prefix(__builtin_popcount(cmask), nch_total);
-    if (sp + nch_total > kLoneStack) {
-      if (lane == 0) atomicOr(err, 1u);
-      return;
+    // offsets of the children (child 0 of every lane first) and of the lists
+    uint64_t cm[4];
+    int nch = 0;
+    int at[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      cm[k] = ballot((cmask >> k) & 1);
+      at[k] = nch + lanes_before(cm[k]);
+      nch += __builtin_popcountll(cm[k]);
     }
-    for (int k = 0; k < 4; ++k)
-      if ((cmask >> k) & 1) s_cell[at++] = child + k;
-    sp += nch_total;
-    // particle lists: the opened leaves and the near big lists of this pop
-    int nref = 0, np = 0;
-    const bool has = pkind >= 0 && pcnt > 0;
-    const int ri = wave_prefix(has ? 1 : 0, nref);
-    const int pre = wave_prefix(has ? pcnt : 0, np);
-    if (has) {
-      s_pst[ri] = pst;
-      s_pcnt[ri] = pcnt;
-      s_pkind[ri] = pkind;
-      s_pre[ri] = pre;
-    }
-    __syncthreads();
-    for (int q = lane; q < np; q += kWave) {
-      int lo = 0, hi = nref - 1;   // the last list whose prefix is <= q
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (s_pre[mid] <= q) lo = mid;
-        else hi = mid - 1;
+    const int scan = wave_scan(pcnt);
+    int np = uni(__builtin_amdgcn_readlane(scan, 63));
+    int pre = scan - pcnt, choff = sp, npall = np;
+    nch = uni(nch);
+    if (NW > 1) {
+      if (lane == 0) {
+        s.nch[w] = nch;
+        s.np[w] = np;
       }
-      const int idx = s_pst[lo] + (q - s_pre[lo]);
-      const int kind = s_pkind[lo];
-      if (kind == 2) {
-        // an internal cell's big particle: its B-spline correction
-        const PartD p = bigs[idx];
-        const double d0 = p.x - rx, d1 = p.y - ry;
-        double rr = d0 * d0 + d1 * d1;
-        if (rr < 1e-20) rr = 1e-20;
-        const double size = p.h;
-        if (rr < 4 * size * size)
-          bspline64(d0, d1, sqrt(rr), (double)p.m, size, a.ax, a.ay, a.k, a.g0, a.g1);
-      } else {
-        // a leaf particle as a point mass (include/quadTree.h:1014-1048),
-        // and its B-spline correction when it is big and the leaf near
-        const PartD p = parts[idx];
-        const double d0 = p.x - rx, d1 = p.y - ry;
-        double rr = d0 * d0 + d1 * d1;
-        if (rr < 1e-20) rr = 1e-20;
-        const double m = p.m;
-        const double inv = rcp64(rr);
-        const double pref = m * inv * kInvPI;
-        a.ax += (ia * m - pref) * d0;
-        a.ay += (ia * m - pref) * d1;
-        const double tmp = -2.0 * pref * inv;
-        a.g0 += 0.5 * (d0 * d0 - d1 * d1) * tmp;
-        a.g1 += d0 * d1 * tmp;
-        a.k -= m * ia;
-        if (kind == 1 && !signbit(p.h)) {
-          const double size = p.h;
-          if (rr < 4 * size * size)
-            bspline64(d0, d1, sqrt(rr), (double)p.m, size, a.ax, a.ay, a.k, a.g0, a.g1);
+      __syncthreads();   // also: the stack entries are read
+      nch = npall = 0;
+      for (int v = 0; v < NW; ++v) {
+        if (v < w) {
+          choff += s.nch[v];
+          pre += s.np[v];
         }
+        nch += s.nch[v];
+        npall += s.np[v];
       }
+    } else {
+      __syncthreads();
     }
-    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if ((cmask >> k) & 1) s.cell[choff + at[k]] = child + k;
+    sp += uni(nch);
+    npall = uni(npall);
+    if (npall <= NW * kLoneItems) {
+      for (int k = 0; ballot(k < pcnt) != 0; ++k)
+        if (k < pcnt) {
+          s.item[pre + k] = (uint32_t)(pst + k);
+          s.kind[pre + k] = (uint8_t)pkind;
+        }
+      __syncthreads();
+      for (int q = tid; q < npall; q += NW * kWave) {
+        const int kind = s.kind[q];
+        const uint32_t idx = s.item[q];
+        lone_particle((kind == 2 ? bigs : parts)[idx], kind, rx, ry, ia, a);
+      }
+    } else {
+      // coarse leaves (a large bucket, or a maximum range): list by list
+      uint64_t m = ballot(pcnt > 0);
+      while (m) {
+        const int l = __builtin_ctzll(m);
+        m &= m - 1;
+        const int st = __builtin_amdgcn_readlane(pst, l), n = __builtin_amdgcn_readlane(pcnt, l);
+        const int kind = __builtin_amdgcn_readlane(pkind, l);
+        for (int k = lane; k < n; k += kWave)
+          lone_particle((kind == 2 ? bigs : parts)[st + k], kind, rx, ry, ia, a);
+      }
+      __syncthreads();
+    }
   }
 }
 
 }  // namespace
 
-// jobs[0]'s plane step for the rays at slots 0 .. nrays-1 (dense state), one
-// wavefront (block) per ray; planes of particle trees only.
-__global__ __launch_bounds__(kWave) void k_plane_step_lone(const StepJob* __restrict__ jobs,
-                                                          uint32_t nrays,
-                                                          uint32_t* __restrict__ err) {
-  __shared__ int32_t s_cell[kLoneStack];
-  __shared__ int32_t s_pst[kWave], s_pcnt[kWave], s_pkind[kWave], s_pre[kWave];
+// A plane step of each listed ray (items == null: rays 0 .. nitems - 1 of
+// jobs[0]; slot = ray, dense state), one block of NW wavefronts per ray; planes
+// of particle trees only.
+template <int NW>
+__global__ __launch_bounds__(NW* kWave) void k_plane_step_lone(const StepJob* __restrict__ jobs,
+                                                              const WorkItem* __restrict__ items,
+                                                              uint32_t nitems) {
+  __shared__ LoneShared<NW> s;
   const uint32_t r = xcd_block(blockIdx.x, gridDim.x);
-  if (r >= nrays) return;
-  const StepJob jb = as_const(jobs)[0];
-  const int slot = (int)r;
+  if (r >= nitems) return;
+  WorkItem it{0u, r};
+  if (items) {
+    it.job = as_const(items)[r].job;
+    it.bundle = as_const(items)[r].bundle;
+  }
+  const StepJob jb = as_const(jobs)[it.job];
+  const int slot = (int)it.bundle;
   const RayState st = state_view(jb.sbase, jb.nslots);
   if (jb.j >= st.jmax[slot]) return;
   const double rx = phys_coord(st.th0[slot], jb.Dphys), ry = phys_coord(st.th1[slot], jb.Dphys);
-  double alpha0 = 0, alpha1 = 0, kappa = 0, gamma0 = 0, gamma1 = 0;
+  double tot[5] = {0, 0, 0, 0, 0};
   const int ntrees = uni(jb.ntrees);
+  const int w = uni((int)threadIdx.x >> 6);
   for (int h = 0; h < ntrees; ++h) {
     const TreeDesc t = as_const(jb.trees)[h];
     Acc64 a;
-    lone_walk64(t, rx, ry, a, s_cell, s_pst, s_pcnt, s_pkind, s_pre, err);
-    alpha0 += wave_sum(a.ax);
-    alpha1 += wave_sum(a.ay);
-    kappa += wave_sum(a.k);
-    gamma0 += wave_sum(a.g0);
-    gamma1 += wave_sum(a.g1);
+    lone_walk64<NW>(t, rx, ry, a, s);
+    double v[5] = {a.ax, a.ay, a.k, a.g0, a.g1};
+    for (int k = 0; k < 5; ++k) v[k] = wave_sum(v[k]);
+    if (NW > 1) {
+      if (lane_id() == 0)
+        for (int k = 0; k < 5; ++k) s.sum[w][k] = v[k];
+      __syncthreads();
+      for (int k = 0; k < 5; ++k) {
+        v[k] = s.sum[0][k];
+        for (int u = 1; u < NW; ++u) v[k] += s.sum[u][k];
+      }
+      __syncthreads();
+    }
+    for (int k = 0; k < 5; ++k) tot[k] += v[k];
   }
-  if (lane_id() == 0) recursion_step(jb, slot, alpha0, alpha1, kappa, gamma0, gamma1);
+  if (threadIdx.x == 0) recursion_step(jb, slot, tot[0], tot[1], tot[2], tot[3], tot[4]);
 }
 
 __global__ void k_zero_u32(uint32_t* __restrict__ p, int n) {
@@ -1979,8 +2048,11 @@ void launch_plane_steps_fused(int precision, unsigned nblocks, uint32_t nitems, 
   else launch_fused_hk<0>(precision, nb, nitems, st, jobs, items, counter, err);
 }
 
-void launch_plane_step_lone(hipStream_t st, const StepJob* job, uint32_t nrays, uint32_t* err) {
-  if (nrays > 0) k_plane_step_lone<<<nrays, kWave, 0, st>>>(job, nrays, err);
+void launch_plane_step_lone(hipStream_t st, int waves, const StepJob* jobs, const WorkItem* items,
+                            uint32_t nitems) {
+  if (nitems == 0) return;
+  if (waves == 4) k_plane_step_lone<4><<<nitems, 4 * kWave, 0, st>>>(jobs, items, nitems);
+  else k_plane_step_lone<1><<<nitems, kWave, 0, st>>>(jobs, items, nitems);
 }
 
 void launch_zero_u32(hipStream_t st, uint32_t* p, int n) {

@@ -224,8 +224,21 @@ constexpr double kGuardSmallAlpha = 0.01;
 // the guard's FP64 shoot puts fewer than 64 rays in a bundle while that
 // still leaves at most this many bundles (about the waves the GPU holds)
 constexpr int64_t kGuardWaves = 8192;
-// up to this many re-shot rays: one wavefront per ray
+// up to this many re-shot rays: the lone-ray walk
 constexpr int64_t kGuardLoneRays = 8192;
+// Lists of up to this many rays go to the lone-ray FP64 walk.  Its time grows
+// with the rays (about 0.045 us a ray and plane), the bundle walk's is its
+// slowest wavefront's however few there are.  Measured, lone against bundles:
+// FP64, two planes of 200,000 particles over 300": 3,000 rays 0.5 / 13 ms,
+// 32,000 rays 2.9 / 7.8 ms, 60,000 rays about 8 ms either way on one
+// 65,536-particle halo's 30"; FP32C, 8,000 rays 0.7 / 2.4 ms on that halo and
+// 1.2 / 14 ms on two planes of 10^6 particles, 32,000 rays 1.9 / 2.5 and
+// 4.2 / 11.7 ms.
+constexpr size_t kLoneRays64 = 49152, kLoneRays32 = 16000;
+// Wavefronts of the lone-ray walk per ray: four while the chip has slots for
+// them.  A call of 1,000 rays through two planes of 10^6 particles: 0.36 ms
+// with four, 0.49 with one; 2,050 rays 0.50 and 0.52; 3,000 rays 0.65 and 0.57.
+inline int lone_waves(int64_t n) { return n <= 2048 ? 4 : 1; }
 
 // A call's slots for the guard kernels: x == null: the tiles of an N x N
 // GridMap; else slot s < n holds ray perm[s] (perm == null: ray s) of x,
@@ -444,9 +457,11 @@ struct FlatLCDM;
 // that walk them)
 void launch_plane_step(int precision, bool count, uint32_t nitems, hipStream_t st,
                        const StepJob* jobs, const WorkItem* items, uint32_t* err, int halos);
-// one plane step (the job at `job`) of the rays at slots 0 .. nrays-1, one
-// wavefront per ray (FP64, planes of particle trees only)
-void launch_plane_step_lone(hipStream_t st, const StepJob* job, uint32_t nrays, uint32_t* err);
+// a plane step of single rays, `waves` (1 or 4) wavefronts each: item i is
+// (job, slot); items == nullptr: slots 0 .. nitems-1 of job 0 (FP64, planes of
+// particle trees only)
+void launch_plane_step_lone(hipStream_t st, int waves, const StepJob* jobs, const WorkItem* items,
+                            uint32_t nitems);
 // every plane step of the listed bundles in one launch, each wavefront taking
 // its bundles through their steps (nblocks == 0: one wavefront per item,
 // else a persistent grid of nblocks blocks on a work queue at `counter`)
@@ -511,6 +526,7 @@ int guard_refine_ctx(slsim_lens L, const RayState& st, int64_t nslots, const Gua
 void uniform_source(const slsim_lens_s* L, double zs, int32_t* jmax, double* aal, double* bbl);
 void make_steps(const slsim_lens_s* L, const RayState& st, int64_t nslots, uint32_t* counters,
                 std::vector<StepJob>& steps);
+bool list_is_lone(const slsim_lens_s* L, size_t n, int precision);
 // GridMap::find_images over a shot grid (images.hip)
 int find_images(slsim_ctx c, const GridGeom& g, const double* y_dev, const double* A_dev,
                 size_t nsrc, const double* ys, size_t cap, int32_t* multiplicity, double* rays,
