@@ -6,11 +6,11 @@
 // source-plane image contains ys (sign tests of three cross products, edges
 // and a vertex included by the reference's rules) yields an image at its
 // centroid (edge midpoint, vertex) with A the mean of its three A matrices.
-// The device tests every (cell, source) pair: one thread per cell keeps its
-// four source-plane corners in registers and runs through the sources staged
-// in LDS; hits are appended per source, then ordered on the host by (cell,
-// triangle), which is the reference's order (rows, then cells, first
-// triangle first), and turned into rays.  The cross products are computed
+// One thread per cell tests the sources, binned over their extent, near its two
+// triangles, and whole workgroups test the triangles that cover many; hits are
+// appended per source, then ordered on the host by (cell, triangle), which is
+// the reference's order (rows, then cells, first triangle first), and turned
+// into rays.  The cross products are computed
 // without FMA contraction, as the reference's, so every sign decision and
 // every image is the reference's to the bit.
 
@@ -131,6 +131,87 @@ __device__ inline void add_hit(uint32_t* count, ImageHit* hits, uint32_t cap, in
   if (at < cap) hits[(int64_t)s * cap + at] = {cell, code};
 }
 
+// A triangle of the grid in the source plane (cell k's first or second).
+struct Tri {
+  int64_t k;
+  int t;
+  double ax, ay, bx, by, cx, cy;
+  bool finite;
+};
+
+__device__ inline Tri load_tri(const double* __restrict__ y, int64_t nx, int64_t k, int t) {
+  const int64_t kb = k + nx + 1, kc = t == 0 ? k + 1 : k + nx;
+  Tri r{k, t, y[2 * k], y[2 * k + 1], y[2 * kb], y[2 * kb + 1], y[2 * kc], y[2 * kc + 1], false};
+  r.finite = isfinite(r.ax) && isfinite(r.ay) && isfinite(r.bx) && isfinite(r.by) &&
+             isfinite(r.cx) && isfinite(r.cy);
+  return r;
+}
+
+// the bins that a finite triangle's bounding box covers, widened by one each
+// side; false: none
+struct BinBox {
+  int x0, x1, y0, y1;
+};
+__device__ inline bool bin_box(const SourceBins& b, const Tri& r, BinBox* o) {
+#pragma clang fp contract(off)
+  const double top = (double)(b.G - 1);
+  const double fx0 = (fmin(fmin(r.ax, r.bx), r.cx) - b.x0) * b.inv_w;
+  const double fx1 = (fmax(fmax(r.ax, r.bx), r.cx) - b.x0) * b.inv_w;
+  const double fy0 = (fmin(fmin(r.ay, r.by), r.cy) - b.y0) * b.inv_w;
+  const double fy1 = (fmax(fmax(r.ay, r.by), r.cy) - b.y0) * b.inv_w;
+  if (b.G <= 0 || fx1 < -1.0 || fy1 < -1.0 || fx0 > top + 1.0 || fy0 > top + 1.0) return false;
+  *o = {(int)fmax(floor(fx0) - 1.0, 0.0), (int)fmin(floor(fx1) + 1.0, top),
+        (int)fmax(floor(fy0) - 1.0, 0.0), (int)fmin(floor(fy1) + 1.0, top)};
+  return true;
+}
+
+// the images a triangle makes of the sources, appended per source
+struct Hits {
+  uint32_t* count;
+  ImageHit* hits;
+  uint32_t cap;
+};
+__device__ inline void test_source(const Tri& r, double q0, double q1, int32_t s, const Hits& h) {
+  const int cd = tri_code(q0, q1, r.ax, r.ay, r.bx, r.by, r.cx, r.cy, r.t == 0);
+  if (cd >= 0)
+    add_hit(h.count, h.hits, h.cap, s, (uint32_t)r.k, ((uint32_t)cd << 1) | (uint32_t)r.t);
+}
+
+// rows row0, row0 + rows, ... of the box, sources from, from + step, ... of each
+__device__ inline void test_box(const Tri& r, const BinBox& o, const SourceBins& b, int row0,
+                                int rows, int from, int step, const Hits& h) {
+  for (int by = o.y0 + row0; by <= o.y1; by += rows) {
+    const int32_t e = b.start[by * b.G + o.x1 + 1];
+    for (int32_t q = b.start[by * b.G + o.x0] + from; q < e; q += step) {
+      const double2 sq = b.sy[q];
+      test_source(r, sq.x, sq.y, b.src[q], h);
+    }
+  }
+}
+
+// Triangles with more than kManySources sources, or kManyRows rows of bins, to
+// test are left to whole workgroups.  A cell by a point mass is mapped over
+// much of the source plane: alone, its lane tested thousands of sources one
+// after the other and the search waited for it.  10,000 sources on 1024^2
+// points: 8.71 -> 4.02 ms a call.  The line lies above what an ordinary cell
+// has in its bins (up to 160 here): at 48 sources and 8 rows the queue
+// overflows and the call takes 9.2 ms.
+constexpr int kManySources = 512, kManyRows = 16;
+constexpr uint32_t kTriQueue = 1u << 18;   // triangles left; beyond: tested where found
+constexpr int kTriBlocks = 2048;
+struct TriQueue {
+  uint64_t* tri;       // 2 cell + triangle
+  uint32_t* count;
+  uint32_t cap;
+};
+__device__ inline bool leave(const TriQueue& queue, const Tri& r) {
+  if (queue.cap == 0) return false;
+  const uint32_t at = atomicAdd(queue.count, 1u);
+  if (at >= queue.cap) return false;
+  queue.tri[at] = 2 * (uint64_t)r.k + (uint64_t)r.t;
+  return true;
+}
+
 // One thread per cell; each of its two triangles tests the sources in the
 // bins its source-plane bounding box covers (widened by a bin each side); a
 // source outside that box fails the sign tests unless the triangle is
@@ -139,52 +220,54 @@ __device__ inline void add_hit(uint32_t* count, ImageHit* hits, uint32_t cap, in
 // the non-finite sources, as the reference's all-pairs search does.
 __global__ __launch_bounds__(256) void k_find_images(const double* __restrict__ y, int64_t nx,
                                                      int64_t ny, const double* __restrict__ ys,
-                                                     int nsrc, SourceBins b, uint32_t cap,
-                                                     uint32_t* __restrict__ count,
-                                                     ImageHit* __restrict__ hits) {
-#pragma clang fp contract(off)
+                                                     int nsrc, SourceBins b, Hits h,
+                                                     TriQueue queue) {
   const int64_t ncell = (nx - 1) * (ny - 1);
   const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (c >= ncell) return;
   const int64_t k = (c / (nx - 1)) * nx + c % (nx - 1);
-  const double p0x = y[2 * k], p0y = y[2 * k + 1];
-  const double p1x = y[2 * (k + nx + 1)], p1y = y[2 * (k + nx + 1) + 1];
   for (int t = 0; t < 2; ++t) {
-    const int64_t k2 = t == 0 ? k + 1 : k + nx;
-    const double p2x = y[2 * k2], p2y = y[2 * k2 + 1];
-    const uint32_t code0 = (uint32_t)t;
-    const bool first = t == 0;
-    const bool finite = isfinite(p0x) && isfinite(p0y) && isfinite(p1x) && isfinite(p1y) &&
-                        isfinite(p2x) && isfinite(p2y);
-    if (!finite) {
-      for (int s = 0; s < nsrc; ++s) {
-        const int cd = tri_code(ys[2 * s], ys[2 * s + 1], p0x, p0y, p1x, p1y, p2x, p2y, first);
-        if (cd >= 0) add_hit(count, hits, cap, s, (uint32_t)k, ((uint32_t)cd << 1) | code0);
-      }
+    const Tri r = load_tri(y, nx, k, t);
+    if (!r.finite) {
+      if (!leave(queue, r))
+        for (int s = 0; s < nsrc; ++s) test_source(r, ys[2 * s], ys[2 * s + 1], s, h);
       continue;
     }
-    const double top = (double)(b.G - 1);
-    const double fx0 = (fmin(fmin(p0x, p1x), p2x) - b.x0) * b.inv_w;
-    const double fx1 = (fmax(fmax(p0x, p1x), p2x) - b.x0) * b.inv_w;
-    const double fy0 = (fmin(fmin(p0y, p1y), p2y) - b.y0) * b.inv_w;
-    const double fy1 = (fmax(fmax(p0y, p1y), p2y) - b.y0) * b.inv_w;
-    if (b.G > 0 && !(fx1 < -1.0 || fy1 < -1.0 || fx0 > top + 1.0 || fy0 > top + 1.0)) {
-      const int bx0 = (int)fmax(floor(fx0) - 1.0, 0.0), bx1 = (int)fmin(floor(fx1) + 1.0, top);
-      const int by0 = (int)fmax(floor(fy0) - 1.0, 0.0), by1 = (int)fmin(floor(fy1) + 1.0, top);
-      for (int by = by0; by <= by1; ++by) {
-        const int32_t e = b.start[by * b.G + bx1 + 1];
-        for (int32_t q = b.start[by * b.G + bx0]; q < e; ++q) {
-          const double2 sq = b.sy[q];
-          const int cd = tri_code(sq.x, sq.y, p0x, p0y, p1x, p1y, p2x, p2y, first);
-          if (cd >= 0) add_hit(count, hits, cap, b.src[q], (uint32_t)k, ((uint32_t)cd << 1) | code0);
-        }
+    BinBox o;
+    if (bin_box(b, r, &o)) {
+      bool many = o.y1 - o.y0 >= kManyRows;
+      if (!many) {
+        int n = 0;
+        for (int by = o.y0; by <= o.y1; ++by)
+          n += b.start[by * b.G + o.x1 + 1] - b.start[by * b.G + o.x0];
+        many = n > kManySources;
       }
+      if (!many || !leave(queue, r)) test_box(r, o, b, 0, 1, 0, 1, h);
     }
     for (int32_t q = 0; q < b.nodd; ++q) {
       const int32_t s = b.odd[q];
-      const int cd = tri_code(ys[2 * s], ys[2 * s + 1], p0x, p0y, p1x, p1y, p2x, p2y, first);
-      if (cd >= 0) add_hit(count, hits, cap, s, (uint32_t)k, ((uint32_t)cd << 1) | code0);
+      test_source(r, ys[2 * s], ys[2 * s + 1], s, h);
     }
+  }
+}
+
+// The triangles left: one workgroup each, a wavefront per row of bins, a lane
+// per source (neighbouring sources are consecutive, so its loads are whole
+// lines).  The hits are ordered on the host, so their order here is free.
+__global__ __launch_bounds__(256) void k_find_images_many(const double* __restrict__ y,
+                                                          int64_t nx,
+                                                          const double* __restrict__ ys, int nsrc,
+                                                          SourceBins b, Hits h, TriQueue queue) {
+  const uint32_t n = min(*queue.count, queue.cap);
+  for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+    const uint64_t e = queue.tri[i];
+    const Tri r = load_tri(y, nx, (int64_t)(e >> 1), (int)(e & 1));
+    if (!r.finite) {
+      for (int s = threadIdx.x; s < nsrc; s += 256) test_source(r, ys[2 * s], ys[2 * s + 1], s, h);
+      continue;
+    }
+    BinBox o;
+    if (bin_box(b, r, &o)) test_box(r, o, b, threadIdx.x >> 6, 4, threadIdx.x & 63, 64, h);
   }
 }
 
@@ -327,9 +410,18 @@ int find_images(slsim_ctx c, const GridGeom& g, const double* y_dev, const doubl
   bins.y0 = by0;
   bins.inv_w = inv_w;
   const int64_t ncell = (g.nx - 1) * (g.ny - 1);
+  // (with no more than kManySources sources no triangle has more to test)
+  TriQueue queue{nullptr, nullptr, 0};
+  if (nsrc > (size_t)kManySources) {
+    queue.cap = (uint32_t)std::min<int64_t>(kTriQueue, 2 * ncell);
+    if ((rc = sc.get(&queue.tri, queue.cap)) || (rc = sc.get(&queue.count, 1))) return rc;
+    launch_zero_u32(st, queue.count, 1);
+  }
+  const Hits h{dcount, dhits, (uint32_t)cap};
   k_find_images<<<(unsigned)((ncell + 255) / 256), 256, 0, st>>>(y_dev, g.nx, g.ny, dys,
-                                                                  (int)nsrc, bins, (uint32_t)cap,
-                                                                  dcount, dhits);
+                                                                  (int)nsrc, bins, h, queue);
+  if (queue.cap > 0)
+    k_find_images_many<<<kTriBlocks, 256, 0, st>>>(y_dev, g.nx, dys, (int)nsrc, bins, h, queue);
   SLSIM_HIP_CHECK(hipGetLastError());
   std::vector<uint32_t> cnt(nsrc);
   SLSIM_HIP_CHECK(hipMemcpyAsync(cnt.data(), dcount, 4 * nsrc, hipMemcpyDeviceToHost, st));

@@ -58,3 +58,19 @@ def test_images_cap(shot):
     with pytest.raises(S.SlsimError) as e:
         g.find_images(y[centre], max_per_source=1)
     assert e.value.code == 1
+
+
+@pytest.mark.parametrize("n", [48, 512, 513, 5000])
+def test_images_of_cells_over_many_sources(shot, n):
+    """Triangles with few and with many sources to test (the line lies at 512
+    sources or 16 rows of bins), on both sides of it: even sources, and
+    sources crowded into a few bins beside far ones.  Equal to the oracle's
+    all-pairs search."""
+    g, x, y, A = shot
+    rng = np.random.default_rng(n)
+    lo, span = y.min(0), np.ptp(y, axis=0)
+    even = lo + rng.random((n, 2)) * span
+    crowd = y[rng.integers(0, g.N * g.N)] + rng.normal(size=(n, 2)) * 1e-9
+    crowd[:3] = even[:3]
+    assert _check(g, x, y, A, even, 4096).max() >= 1
+    _check(g, x, y, A, crowd, 4096)
