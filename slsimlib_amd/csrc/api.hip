@@ -859,7 +859,7 @@ int run_steps(slsim_ctx c, const StepJob* djobs, const StepJob* steps, int jmax,
   for (int j = 0; j < jmax; ++j) {
     if (timed) SLSIM_HIP_CHECK(hipEventRecord(ev[2 * j], c->stream));
     if (lone_rays > 0)
-      launch_plane_step_lone(c->stream, lone_waves(lone_rays), djobs + j, nullptr, lone_rays);
+      launch_plane_step_lone(c->stream, djobs + j, nullptr, lone_rays);
     else
       launch_plane_step(precision, count, nbundles, c->stream, djobs + j, nullptr, err,
                         steps[j].nhtrees > 0 ? steps[j].hkind : 0);

@@ -684,25 +684,17 @@ int slsim_server_s::iterate() {
   }
   job0[SLSIM_DIRECT64 + 1] = nj;
   item0[SLSIM_DIRECT64 + 1] = ni;
-  // lists on the lone-ray walk: a whole plane step each, grouped by the
-  // wavefronts their rays take
-  const int lone_w[2] = {1, 4};
-  size_t ljob0[3], litem0[3];
-  for (int g = 0; g < 2; ++g) {
-    ljob0[g] = nj;
-    litem0[g] = ni;
-    for (auto& t : take) {
-      Req* r = t.first;
-      if (!r->lone || t.second == 0 || lone_waves(r->nrays) != lone_w[g]) continue;
-      h_jobs[nj] = r->steps[r->step];
-      const uint32_t local = (uint32_t)(nj - ljob0[g]);
-      for (int64_t b = 0; b < r->nrays; ++b) h_items[ni++] = {local, (uint32_t)b};
-      ++nj;
-      t.second = r->nbundles - r->next_bundle;
-    }
+  // lists on the lone-ray walk: a whole plane step each
+  const size_t ljob0 = nj, litem0 = ni;
+  for (auto& t : take) {
+    Req* r = t.first;
+    if (!r->lone || t.second == 0) continue;
+    h_jobs[nj] = r->steps[r->step];
+    const uint32_t local = (uint32_t)(nj - ljob0);
+    for (int64_t b = 0; b < r->nrays; ++b) h_items[ni++] = {local, (uint32_t)b};
+    ++nj;
+    t.second = r->nbundles - r->next_bundle;
   }
-  ljob0[2] = nj;
-  litem0[2] = ni;
   SLSIM_HIP_CHECK(hipMemcpyAsync(d_jobs.p, h_jobs, sizeof(StepJob) * nj, hipMemcpyHostToDevice,
                                  stream));
   SLSIM_HIP_CHECK(hipMemcpyAsync(d_items.p, h_items, sizeof(WorkItem) * ni, hipMemcpyHostToDevice,
@@ -718,10 +710,8 @@ int slsim_server_s::iterate() {
                       static_cast<WorkItem*>(d_items.p) + item0[prec],
                       static_cast<uint32_t*>(d_err.p), halos);
   }
-  for (int g = 0; g < 2; ++g)
-    launch_plane_step_lone(stream, lone_w[g], static_cast<StepJob*>(d_jobs.p) + ljob0[g],
-                           static_cast<WorkItem*>(d_items.p) + litem0[g],
-                           (uint32_t)(litem0[g + 1] - litem0[g]));
+  launch_plane_step_lone(stream, static_cast<StepJob*>(d_jobs.p) + ljob0,
+                         static_cast<WorkItem*>(d_items.p) + litem0, (uint32_t)(ni - litem0));
   SLSIM_HIP_CHECK(hipGetLastError());
   // the staging buffers are reused next iteration
   SLSIM_HIP_CHECK(hipStreamSynchronize(stream));

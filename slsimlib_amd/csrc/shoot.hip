@@ -62,9 +62,13 @@ __device__ inline float rcp32(float x) { return __builtin_amdgcn_rcpf(x); }
 #if defined(__HIP_DEVICE_COMPILE__)
 template <typename T>
 using cptr = const __attribute__((address_space(4))) T*;
+template <typename T>
+using lds_ptr = const volatile __attribute__((address_space(3))) T*;
 #else
 template <typename T>
 using cptr = const T*;
+template <typename T>
+using lds_ptr = const volatile T*;
 #endif
 template <typename T>
 __device__ inline cptr<T> as_const(const T* p) {
@@ -88,9 +92,66 @@ struct Counts {
                                                  // leaf-particle iterations
 };
 
-// b_spline_profile (include/quadTree.h:147-190), FP64, phi omitted.
-__device__ inline void bspline64(double d0, double d1, double r, double Mass, double size,
-                                 double& ax, double& ay, double& kap, double& g0, double& g1) {
+struct Acc64 {
+  double ax = 0, ay = 0, k = 0, g0 = 0, g1 = 0;
+};
+
+// The FP64 walk's terms, shared by its bundle and its lone-ray form.  Every
+// rounding is written out (contraction off, FMAs explicit), so that the two
+// forms' sums are equal to the bit whatever code surrounds them.
+
+// A cell's or particle's squared distance.
+__device__ __forceinline__ double dist2(double dx, double dyy) { return fma(dx, dx, dyy); }
+
+// A far cell: monopole + quadrupole (include/quadTree.h:1089-1123).  gamma
+// takes h w and xy w.
+struct Far64 {
+  double ax, ay, h, w, xy;
+};
+__device__ __forceinline__ Far64 far_terms64(const NodeD& nd, double dx, double dy, double dyy,
+                                             double r2, double ia, bool sheet) {
+#pragma clang fp contract(off)
+  Far64 f;
+  const double inv = rcp64(r2);
+  const double mi = nd.mass * inv * kInvPI;
+  const double i2p = inv * inv * kInvPI;
+  const double qx = fma(nd.q2, dy, nd.q0 * dx), qy = fma(nd.q2, dx, nd.q1 * dy);
+  const double qq = fma(dy, qy, dx * qx);
+  const double k = fma(4 * qq * inv, i2p, sheet ? fma(nd.mass, ia, -mi) : -mi);
+  f.ax = fma(k, dx, -(qx * i2p));
+  f.ay = fma(k, dy, -(qy * i2p));
+  f.h = 0.5 * fma(dx, dx, -dyy);
+  f.w = -2.0 * mi * inv;
+  f.xy = dx * dy;
+  return f;
+}
+
+// A leaf particle as a point mass (include/quadTree.h:1014-1048): alpha takes
+// s (d0, d1), gamma h w and xy w.  rr: the squared distance, at least 1e-20.
+struct Point64 {
+  double s, h, w, xy;
+};
+__device__ __forceinline__ Point64 point_terms64(double m, double d0, double d1, double dyy,
+                                                 double rr, double ia, bool sheet) {
+#pragma clang fp contract(off)
+  Point64 t;
+  const double inv = rcp64(rr);
+  const double pref = m * inv * kInvPI;
+  t.s = sheet ? fma(ia, m, -pref) : -pref;
+  t.h = 0.5 * fma(d0, d0, -dyy);
+  t.w = -2.0 * pref * inv;
+  t.xy = d0 * d1;
+  return t;
+}
+
+// b_spline_profile (include/quadTree.h:147-190), FP64, phi omitted: what
+// alpha and gamma lose, and the surface density per mass.  d0d0 = d0 * d0.
+struct Spline64 {
+  double ax, ay, g0, g1, sigma;
+};
+__device__ inline Spline64 bspline_terms64(double d0, double d1, double d0d0, double r,
+                                           double Mass, double size) {
+#pragma clang fp contract(off)
   const double q = r / size;
   double M, sigma;
   if (q > 2) {
@@ -98,27 +159,30 @@ __device__ inline void bspline64(double d0, double d1, double r, double Mass, do
     M = 1;
   } else {
     const double q2 = q * q, q3 = q2 * q;
-    sigma = (8 - 12 * q + 6 * q2 - q3) / 4;
+    sigma = fma(-q, q2, fma(6.0, q2, fma(-12.0, q, 8.0))) / 4;
     if (q > 1) {
       sigma *= 10 / size / size / 7 * kInvPI;
-      M = (-1 + 20 * q2 * (1 - q + 3 * q2 / 8 - q3 / 20)) / 7;
+      M = fma(20 * q2, fma(0.125, 3 * q2, 1 - q) - q3 / 20, -1.0) / 7;
     } else {
-      sigma = 10 * (sigma - 1 + 3 * q - 3 * q2 + q3) / size / size / 7 * kInvPI;
-      M = 10 * q2 * (1 - 3 * q / 4 + 3 * q3 / 10) / 7;
+      sigma = 10 * (fma(-3.0, q2, fma(3.0, q, sigma - 1)) + q3) / size / size / 7 * kInvPI;
+      M = 10 * q2 * (fma(3 * q, -0.25, 1.0) + 3 * q3 / 10) / 7;
     }
   }
   const double alpha_r = (M - 1) * kInvPI / r;
   const double gt = alpha_r / r - sigma;
-  ax -= Mass * alpha_r * d0 / r;
-  ay -= Mass * alpha_r * d1 / r;
-  g0 -= gt * Mass * (d0 * d0 - d1 * d1) / r / r;
-  g1 -= gt * Mass * 2 * d0 * d1 / r / r;
-  kap += Mass * sigma;
+  return {Mass * alpha_r * d0 / r, Mass * alpha_r * d1 / r,
+          gt * Mass * (d0d0 - d1 * d1) / r / r, gt * Mass * 2 * d0 * d1 / r / r, sigma};
 }
-
-struct Acc64 {
-  double ax = 0, ay = 0, k = 0, g0 = 0, g1 = 0;
-};
+__device__ inline void bspline64(double d0, double d1, double d0d0, double r, double Mass,
+                                 double size, Acc64& a) {
+#pragma clang fp contract(off)
+  const Spline64 t = bspline_terms64(d0, d1, d0d0, r, Mass, size);
+  a.ax -= t.ax;
+  a.ay -= t.ay;
+  a.g0 -= t.g0;
+  a.g1 -= t.g1;
+  a.k = fma(Mass, t.sigma, a.k);
+}
 
 // Traversal shared by both walks.  The stack holds opened internal cells as
 // (first child | non-empty-children mask << 28, live mask of the lanes that
@@ -142,6 +206,23 @@ __device__ inline void push_entry(int32_t* s_node, uint64_t* s_mask, int& sp, in
 }
 
 // ---------------------------------------------------------------- FP64 walk
+// A big particle's B-spline correction, where the ray is within 2h.
+template <bool COUNT>
+__device__ __forceinline__ void big_term64(const PartD& p, double rx, double ry, Acc64& a,
+                                           Counts& cnt) {
+#pragma clang fp contract(off)
+  if (COUNT) cnt.b++;
+  const double d0 = p.x - rx, d1 = p.y - ry;
+  const double d0d0 = d0 * d0;
+  double rr = dist2(d1, d0d0);
+  if (rr < 1e-20) rr = 1e-20;
+  const double size = p.h;
+  if (rr < 4 * size * size) {
+    if (COUNT) cnt.s++;
+    bspline64(d0, d1, d0d0, sqrt(rr), (double)p.m, size, a);
+  }
+}
+
 // Evaluates one cell for the lanes with lv set (include/quadTree.h:990-1128):
 // returns the mask of lanes that opened it when it is internal, 0 otherwise.
 // The open test is r^2 < T = max(r2crit, near2) (r^2 < r2crit || r^2 <
@@ -152,8 +233,9 @@ template <bool COUNT>
 __device__ __forceinline__ uint64_t eval64(const NodeD& nd, uint64_t lvm, double rx, double ry,
                                            double ia, cptr<PartD> parts, cptr<PartD> bigs,
                                            Acc64& a, Counts& cnt) {
+#pragma clang fp contract(off)
   const double dx = nd.cx - rx, dy = nd.cy - ry;
-  const double r2 = dx * dx + dy * dy;
+  const double dyy = dy * dy, r2 = dist2(dx, dyy);
   const uint64_t omask = lanes_lt(r2, nd.T) & lvm;
   const bool lv = lane_in(lvm);
   const bool open = lane_in(omask);
@@ -161,44 +243,31 @@ __device__ __forceinline__ uint64_t eval64(const NodeD& nd, uint64_t lvm, double
   if (COUNT) cnt.wv++;
   if (COUNT && lv) cnt.v++;
   if (omask != lvm && lv && !open) {
-    // far cell: monopole + quadrupole (include/quadTree.h:1089-1123)
     if (COUNT) cnt.c++;
-    const double inv = rcp64(r2);
-    const double mi = nd.mass * inv * kInvPI;
-    double tmp = sheet ? nd.mass * ia - mi : -mi;
-    a.ax += tmp * dx;
-    a.ay += tmp * dy;
-    tmp = -2.0 * mi * inv;
-    a.g0 += 0.5 * (dx * dx - dy * dy) * tmp;
-    a.g1 += dx * dy * tmp;
-    const double i2p = inv * inv * kInvPI;
-    a.ax -= (nd.q0 * dx + nd.q2 * dy) * i2p;
-    a.ay -= (nd.q1 * dy + nd.q2 * dx) * i2p;
-    tmp = 4 * (nd.q0 * dx * dx + nd.q1 * dy * dy + 2 * nd.q2 * dx * dy) * inv * i2p;
-    a.ax += tmp * dx;
-    a.ay += tmp * dy;
+    const Far64 f = far_terms64(nd, dx, dy, dyy, r2, ia, sheet);
+    a.ax += f.ax;
+    a.ay += f.ay;
+    a.g0 = fma(f.h, f.w, a.g0);
+    a.g1 = fma(f.xy, f.w, a.g1);
     if (sheet) a.k -= ia * nd.mass;
   }
   const uint64_t om = omask;
   if (om == 0) return 0;
   if (nd.child < 0) {
-    // leaf: every particle as a point mass (include/quadTree.h:1014-1048)
     for (int k = 0; k < nd.count; ++k) {
       const PartD p = parts[nd.start + k];
       if (open) {
         const double d0 = p.x - rx, d1 = p.y - ry;
-        double rr = d0 * d0 + d1 * d1;
+        const double d1d1 = d1 * d1;
+        double rr = dist2(d0, d1d1);
         if (rr < 1e-20) rr = 1e-20;
         const double m = p.m;
-        const double inv = rcp64(rr);
-        const double pref = m * inv * kInvPI;
-        const double s = sheet ? ia * m - pref : -pref;
-        a.ax += s * d0;
-        a.ay += s * d1;
-        const double tmp = -2.0 * pref * inv;
-        a.g0 += 0.5 * (d0 * d0 - d1 * d1) * tmp;
-        a.g1 += d0 * d1 * tmp;
-        if (sheet) a.k -= m * ia;
+        const Point64 t = point_terms64(m, d0, d1, d1d1, rr, ia, sheet);
+        a.ax = fma(t.s, d0, a.ax);
+        a.ay = fma(t.s, d1, a.ay);
+        a.g0 = fma(t.h, t.w, a.g0);
+        a.g1 = fma(t.xy, t.w, a.g1);
+        if (sheet) a.k -= ia * m;
       }
     }
     if (COUNT && open) cnt.p += nd.count;
@@ -209,17 +278,7 @@ __device__ __forceinline__ uint64_t eval64(const NodeD& nd, uint64_t lvm, double
       // the leaf's big particles: h < box (include/quadTree.h:379-396, 1051-1077)
       for (int k = 0; k < nd.count; ++k) {
         const PartD p = parts[nd.start + k];
-        if (nearc && !signbit(p.h)) {
-          if (COUNT) cnt.b++;
-          const double d0 = p.x - rx, d1 = p.y - ry;
-          double rr = d0 * d0 + d1 * d1;
-          if (rr < 1e-20) rr = 1e-20;
-          const double size = p.h;
-          if (rr < 4 * size * size) {
-            if (COUNT) cnt.s++;
-            bspline64(d0, d1, sqrt(rr), (double)p.m, size, a.ax, a.ay, a.k, a.g0, a.g1);
-          }
-        }
+        if (nearc && !signbit(p.h)) big_term64<COUNT>(p, rx, ry, a, cnt);
       }
     }
     return 0;
@@ -230,17 +289,7 @@ __device__ __forceinline__ uint64_t eval64(const NodeD& nd, uint64_t lvm, double
       const bool nearc = lane_in(nm);
       for (int k = 0; k < nd.count; ++k) {
         const PartD p = bigs[nd.start + k];
-        if (nearc) {
-          if (COUNT) cnt.b++;
-          const double d0 = p.x - rx, d1 = p.y - ry;
-          double rr = d0 * d0 + d1 * d1;
-          if (rr < 1e-20) rr = 1e-20;
-          const double size = p.h;
-          if (rr < 4 * size * size) {
-            if (COUNT) cnt.s++;
-            bspline64(d0, d1, sqrt(rr), (double)p.m, size, a.ax, a.ay, a.k, a.g0, a.g1);
-          }
-        }
+        if (nearc) big_term64<COUNT>(p, rx, ry, a, cnt);
       }
     }
   }
@@ -1037,7 +1086,7 @@ __device__ void direct64(const TreeDesc& t, double rx, double ry, bool active, A
     a.g1 += d0 * d1 * tmp;
     a.k -= m * ia;
     const double size = fabs((double)p.h);
-    if (rr < 4 * size * size) bspline64(d0, d1, sqrt(rr), m, size, a.ax, a.ay, a.k, a.g0, a.g1);
+    if (rr < 4 * size * size) bspline64(d0, d1, d0 * d0, sqrt(rr), m, size, a);
   }
 }
 
@@ -1343,37 +1392,73 @@ void k_plane_step_nfw(const StepJob* __restrict__ jobs, const WorkItem* __restri
 }
 
 // ------------------------------------------------------- lone-ray FP64 walk
-// One plane step of one ray by NW wavefronts (one block), for lists of few or
-// scattered rays, where a bundle walk would leave lanes idle and wait on one
-// wavefront's serial traversal: the lanes take the ray's cells NW * 64 at a
-// time from an LDS stack (the last pushed first), a lane that opens an
-// internal cell pushes its children, and the particles of the opened leaves
-// and of the big lists the ray is near are listed in LDS and taken NW * 64 at
-// a time.  The cells, the opening test and the terms are the FP64 walk's
-// (include/quadTree.h:990-1128), so the result is the bundle walk's up to the
-// order of the FP64 sums, which is fixed by the ray and NW alone.
+// One plane step of one ray per wavefront, for lists of few or scattered
+// rays, where a bundle walk would leave lanes idle and wait on one
+// wavefront's serial traversal.  The result is the bundle walk's to the bit:
+// the cells, the opening test and the terms are the same (include/quadTree.h:
+// 990-1128, the functions above), and the sums take the terms in the same
+// order, depth first, a popped entry's children last to first.
 //
-// What bounds it: the latency of a step (LDS stack, cell records from L2,
-// their far terms, the leaf particles' records), about 70 steps of 64 cells a
-// ray on a 2^20-particle plane, so few rays take more wavefronts each
-// (lone_waves) and the LDS is kept small for many rays in flight (10.3 KiB a
-// wavefront; with a 26 KiB stack and a binary search over the leaves for every
-// particle, 0.16 ms a plane of 500,000 particles for some hundred rays, now
-// 0.05).  A list of 40 rays of a 65,536-particle halo takes 0.13 ms (4.0 ms by
-// bundles), 3,001 rays through four planes of 200,000 0.92 ms (30 ms).  A pop takes
-// fewer cells as the stack fills, down to one (depth first, which grows by at
-// most 3 a level), so that the stack never overflows.
+// Two passes over a tree.  The first opens cells breadth first, sixteen
+// entries (64 children, a lane each) at a time, lists the opened cells in LDS
+// and from their subtrees' sizes gives each its depth-first place.  The second
+// takes them in that order, again 64 children at a time: a lane per far cell or
+// listed particle writes the factors of the fused multiply-adds that the bundle
+// walk would do to LDS, and the FP64 matrix instruction runs through them, four
+// a time and all five sums at once.  It is a chain of fused multiply-adds in
+// ascending k (measured equal to the bit on 250,000 sums of random factors,
+// denormals among them; the tests compare whole shoots).
+//
+// A subtree with more opened cells than the list holds is taken apart: its top
+// entry's children are evaluated by themselves, and the opened ones' subtrees
+// go on a stack (a small opening angle; nothing is then too large).
+//
+// What bounds it is the latency of one wavefront's steps.  Of 364,000 cycles a
+// ray on the 65,536-particle halo (880 cells opened, 6,100 terms in 121
+// windows) the opening takes 54,000, the places 19,000, the cells' terms
+// 55,000, the lists and particle loads 66,000, the particles' terms and the
+// writes to LDS 107,000 and the sums 62,000 (286,000 without the reads ahead
+// and with bank conflicts).  11 KB of LDS let 14 rays share a CU; a cap of 128
+// registers for a fourth wavefront a SIMD spilled and gained nothing.  40 rays
+// of that halo take 0.31 ms (4.0 ms by bundles; 0.13 ms with the terms summed
+// by lane, in no fixed order), 3,001 rays through four planes of 200,000
+// 1.41 ms (30 and 0.93 ms).
 namespace {
 
-constexpr int kLoneStack = 1024;    // stack entries per wavefront of the block
-constexpr int kLoneItems = 1280;    // listed particles per wavefront (64 leaves of 20)
-constexpr int kLoneReserve = 3 * (kMaxLevels + 2) + 2;   // what depth-first growth can need
+constexpr int kLoneCells = 1024;   // opened cells listed at a time
+static_assert(kLoneCells <= 8192, "first child and count share 16 bits");
 
-// inclusive scan over the wavefront in registers (DPP row shifts and broadcasts)
+// Factors of a window's terms: alpha's, a common one and one for each
+// component; gamma's, one for each component and a common one; kappa's.  A pass
+// adds kPass terms, which lie so that the eight a lane needs are together
+// (factor_at); the arrays' bases differ mod 8 so that the lanes' reads fall in
+// different banks.  Zeros fill the last pass.
+constexpr int kPass = 32;
+__device__ inline int factor_at(int i) { return (i & ~31) + ((i & 3) << 3) + ((i >> 2) & 7); }
+constexpr int kFacXA = 0, kFacX0 = kWave, kFacX1 = 2 * kWave + 2, kFacG0 = 3 * kWave + 10;
+constexpr int kFacG1 = 4 * kWave + 12, kFacGB = 5 * kWave + 20;
+constexpr int kFacKA = 6 * kWave + 22, kFacKB = 7 * kWave + 30, kLoneFactors = 8 * kWave + 30;
+static_assert(kFacXA % 8 == 0 && kFacG0 % 8 == 2 && kFacG1 % 8 == 4 && kFacKA % 8 == 6, "banks");
+static_assert(kFacX0 % 8 == 0 && kFacX1 % 8 == 2 && kFacGB % 8 == 4 && kFacKB % 8 == 6, "banks");
+
+struct LoneShared {
+  int32_t entry[kLoneCells];       // opened cells: first child | children << 28, breadth first
+  uint16_t kids[kLoneCells];       // index of the first opened child | their number << 13;
+                                   // then the depth-first order
+  union {
+    uint16_t size[kLoneCells];     // opened cells of the subtree; then the place
+    alignas(16) double factor[kLoneFactors];   // of a window's 64 terms
+  };
+  int32_t stack[kStackDepth];
+  uint8_t own[kWave];
+};
+
 template <int CTRL, int ROWS>
 __device__ inline int dpp_or_zero(int v) {
   return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
 }
+// inclusive scans over the wavefront in registers (DPP row shifts and
+// broadcasts): sum, and maximum of values >= 0
 __device__ inline int wave_scan(int v) {
   v += dpp_or_zero<0x111, 0xf>(v);   // row_shr:1
   v += dpp_or_zero<0x112, 0xf>(v);   // row_shr:2
@@ -1383,182 +1468,361 @@ __device__ inline int wave_scan(int v) {
   v += dpp_or_zero<0x143, 0xc>(v);   // row_bcast:31
   return v;
 }
+__device__ inline int wave_scan_max(int v) {
+  v = max(v, dpp_or_zero<0x111, 0xf>(v));
+  v = max(v, dpp_or_zero<0x112, 0xf>(v));
+  v = max(v, dpp_or_zero<0x114, 0xf>(v));
+  v = max(v, dpp_or_zero<0x118, 0xf>(v));
+  v = max(v, dpp_or_zero<0x142, 0xa>(v));
+  v = max(v, dpp_or_zero<0x143, 0xc>(v));
+  return v;
+}
 
 __device__ inline int lanes_before(uint64_t m) {
   return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                         __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
-__device__ inline double wave_sum(double v) {
+// Lists the cells opened below `top` breadth first and leaves their
+// depth-first order in s.kids; returns their number, or -1 when they are more
+// than the list holds (then s.entry[1] on are top's opened children, s.kids[0]
+// their number << 13).
+__device__ int lone_open(const NodeD* __restrict__ nodes, int32_t top, double rx, double ry,
+                         LoneShared& s) {
+#pragma clang fp contract(off)
+  const int lane = lane_id();
+  if (lane == 0) s.entry[0] = top;
+  __syncthreads();
+  int lo = 0, hi = 1, n = 1, nlev = 0;
+  int lev = 0;   // lane l: where level l starts
+  constexpr int kStep = 2;   // loads of sixteen entries' children in flight
+  while (lo < hi) {
+    if (lane == nlev) lev = lo;
+    ++nlev;
+    for (int b = lo; b < hi; b += 16 * kStep) {
+      int32_t opened[kStep];
+      bool open[kStep];
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+      for (int u = 0; u < kStep; ++u) {
+        const int i = b + 16 * u + (lane >> 2);
+        const int32_t e = i < hi ? s.entry[i] : 0;
+        open[u] = (e >> (28 + (lane & 3))) & 1;
+        opened[u] = 0;
+        if (open[u]) {
+          const NodeD& nd = nodes[(e & 0x0fffffff) + (lane & 3)];
+          const double dx = nd.cx - rx, dy = nd.cy - ry;
+          open[u] = dist2(dx, dy * dy) < nd.T && nd.child >= 0;
+          opened[u] = nd.child | (nd.cmask << 28);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kStep; ++u) {
+        const int i = b + 16 * u + (lane >> 2);
+        const uint64_t m = ballot(open[u]);
+        const int c = uni(__builtin_popcountll(m));
+        const int at = n + lanes_before(m);
+        if ((lane & 3) == 0 && i < hi)
+          s.kids[i] = (uint16_t)(at | (__builtin_popcountll((m >> lane) & 0xf) << 13));
+        if (n + c > kLoneCells) {
+          __syncthreads();
+          return -1;
+        }
+        if (open[u]) s.entry[at] = opened[u];
+        n += c;
+      }
+    }
+    __syncthreads();
+    lo = hi;
+    hi = n;
+  }
+  for (int l = nlev - 1; l >= 0; --l) {
+    const int a = __builtin_amdgcn_readlane(lev, l);
+    const int e = l + 1 < nlev ? __builtin_amdgcn_readlane(lev, l + 1) : n;
+    for (int i = a + lane; i < e; i += kWave) {
+      const int kids = s.kids[i], f = kids & 8191, c = kids >> 13;
+      int z[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) z[k] = s.size[k < c ? f + k : 0];
+      int sum = 1;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) sum += k < c ? z[k] : 0;
+      s.size[i] = (uint16_t)sum;
+    }
+    __syncthreads();
+  }
+  if (lane == 0) s.size[0] = 0;
+  __syncthreads();
+  for (int l = 0; l < nlev - 1; ++l) {
+    const int a = __builtin_amdgcn_readlane(lev, l), e = __builtin_amdgcn_readlane(lev, l + 1);
+    for (int i = a + lane; i < e; i += kWave) {
+      const int kids = s.kids[i], f = kids & 8191, c = kids >> 13;
+      int at = s.size[i] + 1, z[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) z[k] = s.size[k < c ? f + k : 0];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (k < c) s.size[f + k] = (uint16_t)at;
+        at += z[k];
+      }
+    }
+    __syncthreads();
+  }
+  for (int i = lane; i < n; i += kWave) s.kids[s.size[i]] = (uint16_t)i;
+  __syncthreads();
+  return n;
 }
 
-// a listed particle: a leaf's as a point mass, with its B-spline correction
-// when it is big and the leaf near (kind 1), or an internal cell's big
-// particle's correction (kind 2)
-__device__ __forceinline__ void lone_particle(const PartD& p, int kind, double rx, double ry,
-                                              double ia, Acc64& a) {
-  const double d0 = p.x - rx, d1 = p.y - ry;
-  double rr = d0 * d0 + d1 * d1;
-  if (rr < 1e-20) rr = 1e-20;
-  const double m = p.m;
-  if (kind != 2) {
-    const double inv = rcp64(rr);
-    const double pref = m * inv * kInvPI;
-    a.ax += (ia * m - pref) * d0;
-    a.ay += (ia * m - pref) * d1;
-    const double tmp = -2.0 * pref * inv;
-    a.g0 += 0.5 * (d0 * d0 - d1 * d1) * tmp;
-    a.g1 += d0 * d1 * tmp;
-    a.k -= m * ia;
-  }
-  if (kind == 2 || (kind == 1 && !signbit(p.h))) {
-    const double size = p.h;
-    if (rr < 4 * size * size) bspline64(d0, d1, sqrt(rr), m, size, a.ax, a.ay, a.k, a.g0, a.g1);
-  }
+// The sums of a wavefront: lane j + 4 b + 16 i holds element (i, j) of the
+// matrix instruction's block b.  Block 0: alpha (j), 1: gamma (i), 2: kappa.
+constexpr int kLaneAx = 0, kLaneAy = 1, kLaneG0 = 4, kLaneG1 = 20, kLaneK = 8;
+
+// Adds a window's n terms to the sums, in order, four a step.
+// All is read ahead; volatile, or the compiler moves the reads to their uses.
+__device__ inline double lone_add(int n, double acc, const LoneShared& s) {
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  const int lane = lane_id(), block = (lane >> 2) & 3, ij = lane & 1, k = (lane >> 4) << 3;
+  const int a = (block == 1 ? (ij ? kFacG1 : kFacG0) : (block == 2 ? kFacKA : kFacXA)) + k;
+  const int b = (block == 1 ? kFacGB : (block == 2 ? kFacKB : (ij ? kFacX1 : kFacX0))) + k;
+  d2 va[2][4], vb[2][4];
+  auto load = [&](int h) {
+    const lds_ptr<d2> pa = (lds_ptr<d2>)(s.factor + a + kPass * h);
+    const lds_ptr<d2> pb = (lds_ptr<d2>)(s.factor + b + kPass * h);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      va[h][u] = pa[u];
+      vb[h][u] = pb[u];
+    }
+  };
+  auto add = [&](int h) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      acc = __builtin_amdgcn_mfma_f64_4x4x4f64(va[h][u].x, vb[h][u].x, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f64_4x4x4f64(va[h][u].y, vb[h][u].y, acc, 0, 0, 0);
+    }
+  };
+  load(0);
+  load(1);
+  __builtin_amdgcn_sched_barrier(0);
+  add(0);
+  if (n > kPass) add(1);
+  return acc;
 }
 
-template <int NW>
-struct LoneShared {
-  int32_t cell[NW * kLoneStack];
-  uint32_t item[NW * kLoneItems];
-  uint8_t kind[NW * kLoneItems];
-  int32_t nch[NW], np[NW];
-  double sum[NW][5];
-};
-
-template <int NW>
-__device__ void lone_walk64(const TreeDesc& t, double rx, double ry, Acc64& a, LoneShared<NW>& s) {
-  const int tid = (int)threadIdx.x, w = uni(tid >> 6), lane = lane_id();
+// The children of the n listed cells, in order, 64 terms a window.  The next
+// window's particles are loaded while a window's terms are added up, the next
+// cells a batch ahead.
+__device__ double lone_eval64(const TreeDesc& t, int n, double rx, double ry, double acc,
+                              LoneShared& s) {
+#pragma clang fp contract(off)
+  const int lane = lane_id(), child = 3 - (lane & 3);
   const NodeD* __restrict__ nodes = t.nodesD;
   const PartD* __restrict__ parts = t.partsD;
   const PartD* __restrict__ bigs = t.bigD;
   const double ia = t.inv_area;
-  constexpr int kCap = NW * kLoneStack;
-  if (tid == 0) s.cell[0] = 0;
+  const bool sheet = ia != 0.0;
+  bool there = false;
+  NodeD nd{};
+  auto load = [&](int k) {
+    const int i = k + (lane >> 2);
+    const int32_t e = i < n ? s.entry[s.kids[i]] : 0;
+    there = (e >> (28 + child)) & 1;
+    if (there) nd = nodes[(e & 0x0fffffff) + child];
+  };
+  load(0);
+  bool kappa_zero = false;   // kappa's factors are zeros
+  // A lane's child of the batch's sixteen cells adds a far cell's term (far),
+  // or a list of particles: a leaf's `cnt`, then their corrections when it is
+  // near (kind 1), or an internal cell's big particles' corrections (kind 2).
+  // pre: where its terms stand in the batch.
+  bool far = false, lists = false;
+  int kind = 0, start = 0, cnt = 0, pre = 0;
+  double mass = 0;
+  Far64 f{};
+  // The window's lane-th term: the q-th of a child's list (o_kind; 0: a far
+  // cell).
+  int o_kind = 0, o_cnt = 0, q = 0, nw = 0;
+  PartD pt{};
+  int total = 0, w0 = 0, k0 = -16;   // the batch's terms, the window, the batch
+  for (bool have = false;; have = true) {
+    bool kappa = sheet;
+    const int nw_now = nw;
+    if (have) {
+      bool spline = false;
+      double ka = 0, kb = 0;
+      const bool mine = lists && lane < nw && o_kind != 0;
+      const int at = factor_at(lane);
+      if (mine) {
+        const double d0 = pt.x - rx, d1 = pt.y - ry;
+        double xa = 0, xb0 = 0, xb1 = 0, ga0 = 0, ga1 = 0, gb = 0;
+        if (o_kind == 1 && q < o_cnt) {
+          const double d1d1 = d1 * d1;
+          double rr = dist2(d0, d1d1);
+          if (rr < 1e-20) rr = 1e-20;
+          const double m = pt.m;
+          const Point64 c = point_terms64(m, d0, d1, d1d1, rr, ia, sheet);
+          xa = c.s;
+          xb0 = d0;
+          xb1 = d1;
+          ga0 = c.h;
+          ga1 = c.xy;
+          gb = c.w;
+          if (sheet) {
+            ka = -(ia * m);
+            kb = 1.0;
+          }
+        } else if (o_kind == 2 || !signbit(pt.h)) {
+          const double d0d0 = d0 * d0;
+          double rr = dist2(d1, d0d0);
+          if (rr < 1e-20) rr = 1e-20;
+          const double size = pt.h;
+          if (rr < 4 * size * size) {
+            const Spline64 c = bspline_terms64(d0, d1, d0d0, sqrt(rr), (double)pt.m, size);
+            xa = -1.0;
+            xb0 = c.ax;
+            xb1 = c.ay;
+            ga0 = c.g0;
+            ga1 = c.g1;
+            gb = -1.0;
+            ka = pt.m;
+            kb = c.sigma;
+            spline = true;
+          }
+        }
+        s.factor[kFacXA + at] = xa;
+        s.factor[kFacX0 + at] = xb0;
+        s.factor[kFacX1 + at] = xb1;
+        s.factor[kFacG0 + at] = ga0;
+        s.factor[kFacG1 + at] = ga1;
+        s.factor[kFacGB + at] = gb;
+      }
+      kappa = kappa || ballot(spline) != 0;
+      const int g = pre - w0, ag = factor_at(g);
+      const bool far_here = far && g >= 0 && g < kWave;
+      if (far_here) {
+        s.factor[kFacXA + ag] = 1.0;
+        s.factor[kFacX0 + ag] = f.ax;
+        s.factor[kFacX1 + ag] = f.ay;
+        s.factor[kFacG0 + ag] = f.h;
+        s.factor[kFacG1 + ag] = f.xy;
+        s.factor[kFacGB + ag] = f.w;
+      }
+      const bool fill = lane >= nw && lane < ((nw + kPass - 1) & ~(kPass - 1));
+      if (fill)
+        s.factor[kFacXA + at] = s.factor[kFacX0 + at] = s.factor[kFacX1 + at] =
+            s.factor[kFacG0 + at] = s.factor[kFacG1 + at] = s.factor[kFacGB + at] = 0.0;
+      if (kappa) {
+        if (mine || fill) {
+          s.factor[kFacKA + at] = ka;
+          s.factor[kFacKB + at] = kb;
+        }
+        if (far_here) {
+          s.factor[kFacKA + ag] = sheet ? -(ia * mass) : 0.0;
+          s.factor[kFacKB + ag] = sheet ? 1.0 : 0.0;
+        }
+        kappa_zero = false;
+      } else if (!kappa_zero) {
+        s.factor[kFacKA + lane] = s.factor[kFacKB + lane] = 0.0;
+        kappa_zero = true;
+      }
+      __syncthreads();
+    }
+    // on to the next window
+    for (w0 += kWave; w0 >= total && k0 < n; w0 = 0) {
+      k0 += 16;
+      total = 0;
+      if (k0 >= n) break;
+      far = false;
+      kind = 0;
+      int terms = 0;
+      if (there) {
+        const double dx = nd.cx - rx, dy = nd.cy - ry;
+        const double dyy = dy * dy, r2 = dist2(dx, dyy);
+        far = !(r2 < nd.T);
+        if (far) {
+          terms = 1;
+          mass = nd.mass;
+          f = far_terms64(nd, dx, dy, dyy, r2, ia, sheet);
+        } else {
+          const bool nearc = r2 < nd.near2;
+          start = nd.start;
+          cnt = nd.count;
+          if (nd.child < 0) {
+            kind = 1;
+            terms = nearc ? 2 * cnt : cnt;
+          } else if (nearc) {
+            kind = 2;
+            terms = cnt;
+          }
+        }
+      }
+      load(k0 + 16);
+      pre = wave_scan(terms) - terms;
+      total = uni(__builtin_amdgcn_readlane(pre + terms, 63));
+      lists = ballot(kind != 0 && terms > 0) != 0;
+    }
+    const bool more = k0 < n;
+    if (more) {
+      nw = total - w0 < kWave ? total - w0 : kWave;
+      if (lists) {
+        // the child that the window's lane-th term belongs to: the last that
+        // starts at or before it
+        s.own[lane] = 0;
+        __syncthreads();
+        const int behind = __shfl_down(pre, 1, kWave);
+        const int end = lane < 63 ? behind : total;
+        if (end > pre && pre < w0 + kWave && end > w0)
+          s.own[pre > w0 ? pre - w0 : 0] = (uint8_t)(lane + 1);
+        __syncthreads();
+        const int o = wave_scan_max(s.own[lane]) - 1;
+        o_kind = __shfl(kind, o, kWave);
+        o_cnt = __shfl(cnt, o, kWave);
+        const int o_start = __shfl(start, o, kWave);
+        q = w0 + lane - __shfl(pre, o, kWave);
+        if (lane < nw && o_kind != 0)
+          pt = (o_kind == 2 ? bigs : parts)[o_start + (q < o_cnt ? q : q - o_cnt)];
+      }
+    }
+    if (have) {
+      acc = lone_add(nw_now, acc, s);
+      __syncthreads();
+    }
+    if (!more) return acc;
+  }
+}
+
+__device__ double lone_walk64(const TreeDesc& t, double rx, double ry, LoneShared& s) {
+  const int lane = lane_id();
+  double acc = 0.0;
+  if (lane == 0) s.stack[0] = 1 << 28;   // the root as the only child of a virtual cell
   int sp = 1;
   __syncthreads();
   while (sp > 0) {
-    // sp + 3 c <= kCap - kLoneReserve, or one cell at a time
-    const int room = (kCap - kLoneReserve - sp) / 3;
-    int c = sp < NW * kWave ? sp : NW * kWave;
-    if (c > room) c = room > 1 ? room : 1;
-    sp -= c;
-    const int cell = tid < c ? s.cell[sp + tid] : -1;
-    int child = 0, cmask = 0, pst = 0, pcnt = 0, pkind = 0;
-    if (cell >= 0) {
-      const NodeD nd = nodes[cell];
-      const double dx = nd.cx - rx, dy = nd.cy - ry;
-      const double r2 = dx * dx + dy * dy;
-      const bool nearc = r2 < nd.near2;
-      if (!(r2 < nd.T)) {
-        // far cell: monopole + quadrupole (include/quadTree.h:1089-1123)
-        const double inv = rcp64(r2);
-        const double mi = nd.mass * inv * kInvPI;
-        double tmp = nd.mass * ia - mi;
-        a.ax += tmp * dx;
-        a.ay += tmp * dy;
-        tmp = -2.0 * mi * inv;
-        a.g0 += 0.5 * (dx * dx - dy * dy) * tmp;
-        a.g1 += dx * dy * tmp;
-        const double i2p = inv * inv * kInvPI;
-        a.ax -= (nd.q0 * dx + nd.q2 * dy) * i2p;
-        a.ay -= (nd.q1 * dy + nd.q2 * dx) * i2p;
-        tmp = 4 * (nd.q0 * dx * dx + nd.q1 * dy * dy + 2 * nd.q2 * dx * dy) * inv * i2p;
-        a.ax += tmp * dx;
-        a.ay += tmp * dy;
-        a.k -= ia * nd.mass;
-      } else if (nd.child < 0) {
-        pst = nd.start;
-        pcnt = nd.count;
-        pkind = nearc ? 1 : 0;
-      } else {
-        child = nd.child;
-        cmask = nd.cmask;
-        if (nearc) {
-          pst = nd.start;
-          pcnt = nd.count;
-          pkind = 2;
-        }
-      }
-    }
-    // offsets of the children (child 0 of every lane first) and of the lists
-    uint64_t cm[4];
-    int nch = 0;
-    int at[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      cm[k] = ballot((cmask >> k) & 1);
-      at[k] = nch + lanes_before(cm[k]);
-      nch += __builtin_popcountll(cm[k]);
-    }
-    const int scan = wave_scan(pcnt);
-    int np = uni(__builtin_amdgcn_readlane(scan, 63));
-    int pre = scan - pcnt, choff = sp, npall = np;
-    nch = uni(nch);
-    if (NW > 1) {
-      if (lane == 0) {
-        s.nch[w] = nch;
-        s.np[w] = np;
-      }
-      __syncthreads();   // also: the stack entries are read
-      nch = npall = 0;
-      for (int v = 0; v < NW; ++v) {
-        if (v < w) {
-          choff += s.nch[v];
-          pre += s.np[v];
-        }
-        nch += s.nch[v];
-        npall += s.np[v];
-      }
-    } else {
+    const int32_t top = uni(s.stack[--sp]);
+    int n = lone_open(t.nodesD, top, rx, ry, s);
+    if (n < 0) {
+      // top by itself, then its opened children's subtrees, the first on top
+      const int c = uni(s.kids[0]) >> 13;
+      if (lane < c) s.stack[sp + c - 1 - lane] = s.entry[1 + lane];
+      sp += c;
       __syncthreads();
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if ((cmask >> k) & 1) s.cell[choff + at[k]] = child + k;
-    sp += uni(nch);
-    npall = uni(npall);
-    if (npall <= NW * kLoneItems) {
-      for (int k = 0; ballot(k < pcnt) != 0; ++k)
-        if (k < pcnt) {
-          s.item[pre + k] = (uint32_t)(pst + k);
-          s.kind[pre + k] = (uint8_t)pkind;
-        }
+      if (lane == 0) s.kids[0] = 0;
       __syncthreads();
-      for (int q = tid; q < npall; q += NW * kWave) {
-        const int kind = s.kind[q];
-        const uint32_t idx = s.item[q];
-        lone_particle((kind == 2 ? bigs : parts)[idx], kind, rx, ry, ia, a);
-      }
-    } else {
-      // coarse leaves (a large bucket, or a maximum range): list by list
-      uint64_t m = ballot(pcnt > 0);
-      while (m) {
-        const int l = __builtin_ctzll(m);
-        m &= m - 1;
-        const int st = __builtin_amdgcn_readlane(pst, l), n = __builtin_amdgcn_readlane(pcnt, l);
-        const int kind = __builtin_amdgcn_readlane(pkind, l);
-        for (int k = lane; k < n; k += kWave)
-          lone_particle((kind == 2 ? bigs : parts)[st + k], kind, rx, ry, ia, a);
-      }
-      __syncthreads();
+      n = 1;
     }
+    acc = lone_eval64(t, n, rx, ry, acc, s);
   }
+  return acc;
 }
 
 }  // namespace
 
 // A plane step of each listed ray (items == null: rays 0 .. nitems - 1 of
-// jobs[0]; slot = ray, dense state), one block of NW wavefronts per ray; planes
-// of particle trees only.
-template <int NW>
-__global__ __launch_bounds__(NW* kWave) void k_plane_step_lone(const StepJob* __restrict__ jobs,
-                                                              const WorkItem* __restrict__ items,
-                                                              uint32_t nitems) {
-  __shared__ LoneShared<NW> s;
+// jobs[0]; slot = ray, dense state), one wavefront per ray; planes of particle
+// trees only.
+__global__ __launch_bounds__(kWave) void k_plane_step_lone(const StepJob* __restrict__ jobs,
+                                                          const WorkItem* __restrict__ items,
+                                                          uint32_t nitems) {
+  __shared__ LoneShared s;
   const uint32_t r = xcd_block(blockIdx.x, gridDim.x);
   if (r >= nitems) return;
   WorkItem it{0u, r};
@@ -1571,28 +1835,16 @@ __global__ __launch_bounds__(NW* kWave) void k_plane_step_lone(const StepJob* __
   const RayState st = state_view(jb.sbase, jb.nslots);
   if (jb.j >= st.jmax[slot]) return;
   const double rx = phys_coord(st.th0[slot], jb.Dphys), ry = phys_coord(st.th1[slot], jb.Dphys);
-  double tot[5] = {0, 0, 0, 0, 0};
+  double tot = 0.0;
   const int ntrees = uni(jb.ntrees);
-  const int w = uni((int)threadIdx.x >> 6);
   for (int h = 0; h < ntrees; ++h) {
     const TreeDesc t = as_const(jb.trees)[h];
-    Acc64 a;
-    lone_walk64<NW>(t, rx, ry, a, s);
-    double v[5] = {a.ax, a.ay, a.k, a.g0, a.g1};
-    for (int k = 0; k < 5; ++k) v[k] = wave_sum(v[k]);
-    if (NW > 1) {
-      if (lane_id() == 0)
-        for (int k = 0; k < 5; ++k) s.sum[w][k] = v[k];
-      __syncthreads();
-      for (int k = 0; k < 5; ++k) {
-        v[k] = s.sum[0][k];
-        for (int u = 1; u < NW; ++u) v[k] += s.sum[u][k];
-      }
-      __syncthreads();
-    }
-    for (int k = 0; k < 5; ++k) tot[k] += v[k];
+    tot += lone_walk64(t, rx, ry, s);
   }
-  if (threadIdx.x == 0) recursion_step(jb, slot, tot[0], tot[1], tot[2], tot[3], tot[4]);
+  const double alpha0 = __shfl(tot, kLaneAx, kWave), alpha1 = __shfl(tot, kLaneAy, kWave);
+  const double gamma0 = __shfl(tot, kLaneG0, kWave), gamma1 = __shfl(tot, kLaneG1, kWave);
+  const double kappa = __shfl(tot, kLaneK, kWave);
+  if (threadIdx.x == 0) recursion_step(jb, slot, alpha0, alpha1, kappa, gamma0, gamma1);
 }
 
 __global__ void k_zero_u32(uint32_t* __restrict__ p, int n) {
@@ -1952,7 +2204,7 @@ __global__ __launch_bounds__(256) void k_direct(const PartD* __restrict__ parts,
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   const bool active = i < n;
   const double rx = active ? rays[2 * i] : 0.0, ry = active ? rays[2 * i + 1] : 0.0;
-  double ax = 0, ay = 0, k = 0, g0 = 0, g1 = 0;
+  Acc64 a;
   for (int64_t base = 0; base < np; base += 256) {
     __syncthreads();
     if (base + threadIdx.x < np) tile[threadIdx.x] = parts[base + threadIdx.x];
@@ -1966,19 +2218,19 @@ __global__ __launch_bounds__(256) void k_direct(const PartD* __restrict__ parts,
       const double m = p.m;
       const double inv = rcp64(rr);
       const double pref = m * inv * kInvPI;
-      ax += (ia * m - pref) * d0;
-      ay += (ia * m - pref) * d1;
+      a.ax += (ia * m - pref) * d0;
+      a.ay += (ia * m - pref) * d1;
       const double tmp = -2.0 * pref * inv;
-      g0 += 0.5 * (d0 * d0 - d1 * d1) * tmp;
-      g1 += d0 * d1 * tmp;
-      k -= m * ia;
+      a.g0 += 0.5 * (d0 * d0 - d1 * d1) * tmp;
+      a.g1 += d0 * d1 * tmp;
+      a.k -= m * ia;
       const double size = fabs((double)p.h);
-      if (rr < 4 * size * size) bspline64(d0, d1, sqrt(rr), m, size, ax, ay, k, g0, g1);
+      if (rr < 4 * size * size) bspline64(d0, d1, d0 * d0, sqrt(rr), m, size, a);
     }
   }
   if (active) {
-    out[5 * i] = ax; out[5 * i + 1] = ay; out[5 * i + 2] = k;
-    out[5 * i + 3] = g0; out[5 * i + 4] = g1;
+    out[5 * i] = a.ax; out[5 * i + 1] = a.ay; out[5 * i + 2] = a.k;
+    out[5 * i + 3] = a.g0; out[5 * i + 4] = a.g1;
   }
 }
 
@@ -2048,11 +2300,9 @@ void launch_plane_steps_fused(int precision, unsigned nblocks, uint32_t nitems, 
   else launch_fused_hk<0>(precision, nb, nitems, st, jobs, items, counter, err);
 }
 
-void launch_plane_step_lone(hipStream_t st, int waves, const StepJob* jobs, const WorkItem* items,
+void launch_plane_step_lone(hipStream_t st, const StepJob* jobs, const WorkItem* items,
                             uint32_t nitems) {
-  if (nitems == 0) return;
-  if (waves == 4) k_plane_step_lone<4><<<nitems, 4 * kWave, 0, st>>>(jobs, items, nitems);
-  else k_plane_step_lone<1><<<nitems, kWave, 0, st>>>(jobs, items, nitems);
+  if (nitems > 0) k_plane_step_lone<<<nitems, kWave, 0, st>>>(jobs, items, nitems);
 }
 
 void launch_zero_u32(hipStream_t st, uint32_t* p, int n) {

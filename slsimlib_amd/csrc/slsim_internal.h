@@ -226,19 +226,22 @@ constexpr double kGuardSmallAlpha = 0.01;
 constexpr int64_t kGuardWaves = 8192;
 // up to this many re-shot rays: the lone-ray walk
 constexpr int64_t kGuardLoneRays = 8192;
-// Lists of up to this many rays go to the lone-ray FP64 walk.  Its time grows
-// with the rays (about 0.045 us a ray and plane), the bundle walk's is its
-// slowest wavefront's however few there are.  Measured, lone against bundles:
-// FP64, two planes of 200,000 particles over 300": 3,000 rays 0.5 / 13 ms,
-// 32,000 rays 2.9 / 7.8 ms, 60,000 rays about 8 ms either way on one
-// 65,536-particle halo's 30"; FP32C, 8,000 rays 0.7 / 2.4 ms on that halo and
-// 1.2 / 14 ms on two planes of 10^6 particles, 32,000 rays 1.9 / 2.5 and
-// 4.2 / 11.7 ms.
-constexpr size_t kLoneRays64 = 49152, kLoneRays32 = 16000;
-// Wavefronts of the lone-ray walk per ray: four while the chip has slots for
-// them.  A call of 1,000 rays through two planes of 10^6 particles: 0.36 ms
-// with four, 0.49 with one; 2,050 rays 0.50 and 0.52; 3,000 rays 0.65 and 0.57.
-inline int lone_waves(int64_t n) { return n <= 2048 ? 4 : 1; }
+// Lists of up to this many rays go to the lone-ray walk.  Its time grows with
+// the rays, the bundle walk's is its slowest wavefront's however few there are.
+// FP64 results are the same to the bit either way, so the line lies where the
+// bundles catch up on the lists that suit them best, clustered ones.  Wall ms of
+// a call, lone / bundles, lists over 0.02 of the field and over all of it:
+//   65,536-particle halo, 30":        16,000 rays 1.97 / 2.26 and 1.41 / 3.71,
+//                                     20,000 rays 2.38 / 2.28 and 1.70 / 3.47
+//   two planes of 200,000, 300":      20,000 rays 2.76 / 3.16 and 2.62 / 10.5
+//   two planes of 2^20, 300":         20,000 rays 4.34 / 4.50 and 4.02 / 20.2
+// (square grids of rays as lists are like the second of each).  SLSIM_FP32C:
+// such lists are shot in FP64, which leaves nothing to guard; clustered ones
+// break even with the FP32C bundles at 19,000 to 22,000 rays too (20,000: 2.40
+// / 2.40, 2.75 / 3.12, 4.36 / 4.56), but results change there (FP64 below, the
+// FP32C GridMap's to the bit above), and lists as long as a 128 x 128 grid's
+// keep the GridMap's.
+constexpr size_t kLoneRays64 = 20000, kLoneRays32 = 16000;
 
 // A call's slots for the guard kernels: x == null: the tiles of an N x N
 // GridMap; else slot s < n holds ray perm[s] (perm == null: ray s) of x,
@@ -457,10 +460,10 @@ struct FlatLCDM;
 // that walk them)
 void launch_plane_step(int precision, bool count, uint32_t nitems, hipStream_t st,
                        const StepJob* jobs, const WorkItem* items, uint32_t* err, int halos);
-// a plane step of single rays, `waves` (1 or 4) wavefronts each: item i is
-// (job, slot); items == nullptr: slots 0 .. nitems-1 of job 0 (FP64, planes of
-// particle trees only)
-void launch_plane_step_lone(hipStream_t st, int waves, const StepJob* jobs, const WorkItem* items,
+// a plane step of single rays, a wavefront each: item i is (job, slot);
+// items == nullptr: slots 0 .. nitems-1 of job 0 (FP64, planes of particle
+// trees only)
+void launch_plane_step_lone(hipStream_t st, const StepJob* jobs, const WorkItem* items,
                             uint32_t nitems);
 // every plane step of the listed bundles in one launch, each wavefront taking
 // its bundles through their steps (nblocks == 0: one wavefront per item,

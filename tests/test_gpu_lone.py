@@ -1,6 +1,6 @@
 """Ray lists on the lone-ray FP64 walk: the sizes where its launch changes
-(four wavefronts a ray, one, the bundle walk beyond), coarse leaves whose
-particles outgrow its list, and big particles, against the oracle.
+(the bundle walk beyond 20,000 rays), coarse leaves and big particles, against
+the oracle and, to the bit, against the grid launch.
 
 Tolerance: the same algorithm in the same precision, sums in another order:
 relative |d alpha| <= 1e-9, |d A| <= 1e-8 (the bounds of the FP64 walk's tests).
@@ -68,3 +68,49 @@ def test_leaves_and_big_particles_match_oracle(ctx, bucket, max_range):
         pos = (rng.random((k, 2)) - 0.5) * W.grid_range(60.0)
         yy, A = lens.rayshooterInternal(pos)
         _check(lens, L, pos, yy, A)
+
+
+def _same(r, y, A):
+    return np.array_equal(r[0], y) and np.array_equal(r[1], A)
+
+
+@pytest.mark.parametrize("N", [1, 6, 8, 45, 46, 90, 127, 141, 142, 222])
+def test_list_is_its_gridmap_to_the_bit(ctx, field, N):
+    """A ray's FP64 result does not depend on the rays beside it: the rays of
+    a GridMap as a list in another order, as two lists, and as a served list
+    (sizes on both sides of every limit of the list's walk)."""
+    lens, _ = field
+    rg = W.grid_range(300.0)
+    g = S.GridMap(lens, N, (0.0, 0.0), rg, S.SLSIM_FP64)
+    x, n = g.positions(), N * N
+    perm = np.random.default_rng(N).permutation(n)
+    y, A = g.y()[perm], g.A()[perm]
+    assert _same(lens.rayshooterInternal(x[perm]), y, A)
+    for part in (slice(0, n // 3), slice(n // 3, n)):
+        if len(x[perm][part]):
+            assert _same(lens.rayshooterInternal(x[perm][part]), y[part], A[part])
+    srv = S.Server(ctx, hbm_budget=1 << 30)
+    r = srv.wait_rays(srv.submit_rays(lens, x[perm], precision=S.SLSIM_FP64), n)
+    srv.close()
+    assert _same(r, y, A)
+
+
+@pytest.mark.parametrize("bucket,max_range,theta", [(1, -1.0, 0.1), (20, -1.0, 0.1),
+                                                    (700, -1.0, 0.1), (20, 0.02, 0.1),
+                                                    (5, -1.0, 0.004), (1, -1.0, 0.5)])
+def test_trees_of_any_form_give_the_grid_bits(ctx, bucket, max_range, theta):
+    """As above on coarse leaves, big particles, a mass sheet and, at the
+    smallest opening angle, more opened cells than the walk lists at a time."""
+    rng = np.random.default_rng(bucket)
+    n = 6000
+    x = np.concatenate([0.05 * rng.normal(size=n), 1.0 + 0.01 * rng.random(n // 2)])
+    y = np.concatenate([0.05 * rng.normal(size=n), 0.01 * rng.random(n // 2)])
+    m = (1e9 * (0.5 + rng.random(x.size))).astype(np.float32)
+    h = (10.0 ** rng.uniform(-6, -0.5, x.size)).astype(np.float32)
+    lens = S.Lens(ctx, 2.0)
+    for z, ia in ((0.5, 0.0), (0.5, 30.0), (1.0, 0.0)):
+        lens.moveinMainHalo(S.LensHaloParticles(ctx, x, y, m, h, z, bucket=bucket, theta=theta,
+                                                inv_area=ia, max_range=max_range))
+    g = S.GridMap(lens, 30, (0.0, 0.0), W.grid_range(60.0), S.SLSIM_FP64)
+    assert _same(lens.rayshooterInternal(g.positions()), g.y(), g.A())
+    lens.close()
