@@ -227,10 +227,12 @@ typedef struct {
  * (FullRange/internal_rayshooter_multi.cpp:53-251; include/lens.h:913-1103).
  * Host buffers: x (2n, x0 x1 interleaved, radians), zs (n source redshifts or
  * NULL = lens source), y (2n out), A (4n out, row-major a0 a1 a2 a3).
- * Large lists are Morton-ordered on the device so that each wavefront walks a
- * spatially coherent bundle; short lists take a wavefront or more per ray, in
- * FP64 (SLSIM_FP32C too: nothing is then left to guard, n_guarded is 0).
- * Results come back in input order.
+ * Rays are Morton-ordered on the device so that each wavefront walks a
+ * spatially coherent bundle; short SLSIM_FP64 lists take a wavefront per ray.
+ * A ray's result does not depend on that, or on the rays beside it: it is to
+ * the bit what a GridMap with that ray gives (SLSIM_FP32C: as long as the
+ * guard, whose limits are relative to the call's rms deflection, decides
+ * alike).  Results come back in input order.
  */
 int slsim_shoot(slsim_lens lens, size_t n, const double* x, const double* zs, double* y,
                 double* A, int precision, slsim_shoot_stats* stats);

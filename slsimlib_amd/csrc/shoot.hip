@@ -2021,7 +2021,7 @@ __global__ void k_finalize_array(RayState st, int64_t nslots, int64_t n,
 
 // ----------------------------------------------- precision-form guard
 // A call's slots: ray i and its image position.  Grid: the tiles of a
-// GridMap; array: slot s < n holds ray perm[s] of x.
+// GridMap; array: sorted ray k, ray perm[k] of x.
 __device__ inline bool slot_ray(const GuardMap& m, int64_t slot, int64_t* i, double* x0,
                                 double* x1) {
   if (m.x == nullptr) {
@@ -2029,8 +2029,9 @@ __device__ inline bool slot_ray(const GuardMap& m, int64_t slot, int64_t* i, dou
     grid_position(*i, m.N, m.c0, m.c1, m.range, x0, x1);
     return true;
   }
-  if (slot >= m.n) return false;
-  *i = m.perm ? (int64_t)m.perm[slot] : slot;
+  const int64_t k = array_ray_index(slot, m.lanes);
+  if (k < 0 || k >= m.n) return false;
+  *i = m.perm ? (int64_t)m.perm[k] : k;
   *x0 = m.x[2 * *i];
   *x1 = m.x[2 * *i + 1];
   return true;

@@ -14,7 +14,7 @@ from slsimlib_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
 
-LIMIT64, LIMIT32, FOUR_WAVES = 49152, 16000, 2048
+LIMIT64, SPARSE = 20000, 1024   # rays: to the lone walk; FP32C bundles not yet full, per ray of each
 
 
 def _check(lens, L, x, y, A, zs=None):
@@ -36,8 +36,8 @@ def field(ctx):
     return lens, L
 
 
-@pytest.mark.parametrize("n", [1, 63, 64, 65, FOUR_WAVES, FOUR_WAVES + 1, LIMIT32, LIMIT32 + 1,
-                               LIMIT64, LIMIT64 + 1])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, SPARSE, SPARSE + 1, 16000, 16001, LIMIT64,
+                               LIMIT64 + 1, 32 * SPARSE, 32 * SPARSE + 1, 49152, 49153])
 def test_list_sizes_match_oracle(field, n):
     lens, L = field
     rng = np.random.default_rng(n)
@@ -45,10 +45,12 @@ def test_list_sizes_match_oracle(field, n):
     zs = rng.uniform(0.05, 4.0, n) if n % 2 else None
     y, A = lens.rayshooterInternal(x, zs)
     _check(lens, L, x, y, A, zs)
-    st = {}
-    y32, A32 = lens.rayshooterInternal(x, zs, S.SLSIM_FP32C, stats=st)
-    if n <= LIMIT32:                      # FP64 results: nothing to guard
-        assert np.array_equal(y32, y) and np.array_equal(A32, A) and st["n_guarded"] == 0
+    # the precision form within its bound of the FP64 path at every ray
+    y32, A32 = lens.rayshooterInternal(x, zs, S.SLSIM_FP32C)
+    a = np.linalg.norm(x - y, axis=1)
+    scale = np.maximum(a, 1e-3 * np.sqrt(np.mean(a ** 2)))
+    assert (np.linalg.norm(y32 - y, axis=1) <= 1e-5 * scale).all()
+    assert np.abs(A32 - A).max() <= 1e-3
 
 
 @pytest.mark.parametrize("bucket,max_range", [(1, -1.0), (20, -1.0), (700, -1.0), (20, 0.02)])
@@ -114,3 +116,23 @@ def test_trees_of_any_form_give_the_grid_bits(ctx, bucket, max_range, theta):
     g = S.GridMap(lens, 30, (0.0, 0.0), W.grid_range(60.0), S.SLSIM_FP64)
     assert _same(lens.rayshooterInternal(g.positions()), g.y(), g.A())
     lens.close()
+
+
+@pytest.mark.parametrize("N", [2, 8, 31, 32, 33, 45, 46, 64, 126, 127, 222])
+def test_fp32c_list_is_its_gridmap_to_the_bit(ctx, field, N):
+    """The same in the precision form, with the rays its guard shot again: a
+    GridMap, its rays as a list in another order and as a served list, with 1
+    to 64 rays a bundle."""
+    lens, _ = field
+    rg = W.grid_range(300.0)
+    g = S.GridMap(lens, N, (0.0, 0.0), rg, S.SLSIM_FP32C)
+    x, n = g.positions(), N * N
+    perm = np.random.default_rng(N).permutation(n)
+    y, A = g.y()[perm], g.A()[perm]
+    st = {}
+    assert _same(lens.rayshooterInternal(x[perm], precision=S.SLSIM_FP32C, stats=st), y, A)
+    assert st["n_guarded"] == g.stats["n_guarded"]
+    srv = S.Server(ctx, hbm_budget=1 << 30)
+    r = srv.wait_rays(srv.submit_rays(lens, x[perm], precision=S.SLSIM_FP32C), n)
+    srv.close()
+    assert _same(r, y, A)
