@@ -495,6 +495,9 @@ int slsim_batch_destroy(slsim_batch b) {
 }  // extern "C"
 
 // ==================================================================== server
+// rays of a list on the lone-ray walk that the scheduler counts as a bundle
+constexpr int64_t kLoneUnit = 8;
+
 struct slsim_server_s {
   slsim_ctx ctx = nullptr;
   size_t budget = 0, in_use = 0;
@@ -525,7 +528,9 @@ struct slsim_server_s {
     int32_t jmax = 0, step = 0;
     int64_t nbundles = 0, next_bundle = 0;   // progress within plane `step`
     double aal = 0, bbl = 0;
-    bool lone = false;   // ray list on the lone-ray walk, as a call of its own would be
+    // rays of one bundle; of a list on the lone-ray walk (as a call of its own
+    // would be) kLoneUnit rays, a wavefront each
+    int64_t unit = kWave;
     std::vector<StepJob> steps;
     State state = PENDING;
     int status = SLSIM_OK;
@@ -577,7 +582,7 @@ int slsim_server_s::admit(Req* r) {
     slsim_lens_s* L = r->lens;
     if ((rc = L->upload_trees())) return rc;
     const int64_t n = r->nrays;
-    r->lone = list_is_lone(L, (size_t)n, r->precision);
+    if (list_is_lone(L, (size_t)n, r->precision)) r->unit = kLoneUnit;
     const int nplanes = (int)L->plane_redshifts.size() - 1;
     double* p = reinterpret_cast<double*>(base + ((sbytes + 255) & ~(size_t)255));
     r->xd = p;   p += 2 * n;
@@ -599,7 +604,7 @@ int slsim_server_s::admit(Req* r) {
       else uniform_source(L, 0.0, &r->jmax, &r->aal, &r->bbl);
     }
     make_steps(L, r->st, r->nslots, nullptr, r->steps);
-    r->nbundles = r->nslots / kWave;
+    r->nbundles = (n + r->unit - 1) / r->unit;
     r->next_bundle = 0;
     FlatLCDM cosmo{L->Om, L->OL, L->h};
     launch_init_array(stream, r->st, r->nslots, n, nullptr, r->xd, nplanes > 0 ? r->zsd : nullptr,
@@ -627,7 +632,12 @@ int slsim_server_s::admit(Req* r) {
 // the rest goes to the requests with the least remaining work first.  A
 // request takes bundles of its current plane only; its rays are independent,
 // so how its bundles are split over iterations does not change a bit of its
-// result.  One launch per precision.
+// result.  One launch per precision, and one for the lists on the lone-ray
+// walk, which count kLoneUnit rays as a bundle: on a full chip a ray takes 0.06
+// us a plane of 200,000 particles, a GridMap's bundle 0.4.  (Served lists are
+// not sorted, so full bundles of them are no alternative: 40 lists of 16,000
+// rays through two such planes take 73 ms by lone rays, 171 ms by bundles; ten
+// beside two 1024^2 GridMaps 51 and 254 ms.)
 constexpr int64_t kIterBundles = 32768;
 
 int slsim_server_s::iterate() {
@@ -663,7 +673,8 @@ int slsim_server_s::iterate() {
     left -= t;
   }
   size_t nit = 0;
-  for (auto& t : take) nit += t.first->lone ? (size_t)t.first->nrays : (size_t)t.second;
+  for (auto& t : take)
+    nit += (size_t)(t.first->unit == kWave ? t.second : t.second * kLoneUnit);
   int rc = stage(take.size(), nit);
   if (rc) return rc;
   // jobs and items of all precisions in one staging copy, grouped by precision
@@ -674,7 +685,7 @@ int slsim_server_s::iterate() {
     item0[prec] = ni;
     for (auto& t : take) {
       Req* r = t.first;
-      if (r->lone || r->precision != prec || t.second == 0) continue;
+      if (r->unit != kWave || r->precision != prec || t.second == 0) continue;
       h_jobs[nj] = r->steps[r->step];
       const uint32_t local = (uint32_t)(nj - job0[prec]);
       for (int64_t b = 0; b < t.second; ++b)
@@ -684,16 +695,15 @@ int slsim_server_s::iterate() {
   }
   job0[SLSIM_DIRECT64 + 1] = nj;
   item0[SLSIM_DIRECT64 + 1] = ni;
-  // lists on the lone-ray walk: a whole plane step each
-  const size_t ljob0 = nj, litem0 = ni;
+  const size_t ljob0 = nj, litem0 = ni;   // lists on the lone-ray walk
   for (auto& t : take) {
     Req* r = t.first;
-    if (!r->lone || t.second == 0) continue;
+    if (r->unit == kWave || t.second == 0) continue;
     h_jobs[nj] = r->steps[r->step];
     const uint32_t local = (uint32_t)(nj - ljob0);
-    for (int64_t b = 0; b < r->nrays; ++b) h_items[ni++] = {local, (uint32_t)b};
+    const int64_t end = std::min(r->nrays, kLoneUnit * (r->next_bundle + t.second));
+    for (int64_t k = kLoneUnit * r->next_bundle; k < end; ++k) h_items[ni++] = {local, (uint32_t)k};
     ++nj;
-    t.second = r->nbundles - r->next_bundle;
   }
   SLSIM_HIP_CHECK(hipMemcpyAsync(d_jobs.p, h_jobs, sizeof(StepJob) * nj, hipMemcpyHostToDevice,
                                  stream));

@@ -136,3 +136,23 @@ def test_fp32c_list_is_its_gridmap_to_the_bit(ctx, field, N):
     r = srv.wait_rays(srv.submit_rays(lens, x[perm], precision=S.SLSIM_FP32C), n)
     srv.close()
     assert _same(r, y, A)
+
+
+def test_server_counts_the_rays_of_its_lists(ctx, field):
+    """A scheduler iteration takes up to 32,768 bundles' worth of work, eight
+    rays of a short FP64 list counting as one (it takes a wavefront per ray):
+    40 lists of 16,000 rays through three planes are more than seven
+    iterations' worth.  Their results are the lone call's to the bit, split over
+    iterations as they are."""
+    lens, _ = field
+    rng = np.random.default_rng(40)
+    n, lists, planes = 16000, 40, 3
+    x = (rng.random((n, 2)) - 0.5) * W.grid_range(300.0)
+    ref = lens.rayshooterInternal(x)
+    srv = S.Server(ctx, hbm_budget=1 << 30)
+    ids = [srv.submit_rays(lens, x, precision=S.SLSIM_FP64) for _ in range(lists)]
+    out = [srv.wait_rays(i, n) for i in ids]
+    iterations = srv.stats()["iterations"]
+    srv.close()
+    assert all(_same(ref, y, A) for y, A, _ in out)
+    assert iterations * 32768 >= lists * planes * (n // 8)
