@@ -61,16 +61,119 @@ def test_images_cap(shot):
 
 
 @pytest.mark.parametrize("n", [48, 512, 513, 5000])
-def test_images_of_cells_over_many_sources(shot, n):
-    """Triangles with few and with many sources to test (the line lies at 512
-    sources or 16 rows of bins), on both sides of it: even sources, and
-    sources crowded into a few bins beside far ones.  Equal to the oracle's
-    all-pairs search."""
+def test_images_of_many_sources(shot, n):
+    """Sources over the whole source plane, and sources around the grid's own
+    source positions, in numbers on both sides of the line (512 sources) from
+    which triangles can be left to whole workgroups.  None has that many to test
+    here.  Equal to the oracle's all-pairs search."""
     g, x, y, A = shot
     rng = np.random.default_rng(n)
     lo, span = y.min(0), np.ptp(y, axis=0)
     even = lo + rng.random((n, 2)) * span
-    crowd = y[rng.integers(0, g.N * g.N)] + rng.normal(size=(n, 2)) * 1e-9
-    crowd[:3] = even[:3]
+    near = y[rng.integers(0, g.N * g.N)] + rng.normal(size=(n, 2)) * 1e-9
+    near[:3] = even[:3]
     assert _check(g, x, y, A, even, 4096).max() >= 1
-    _check(g, x, y, A, crowd, 4096)
+    _check(g, x, y, A, near, 4096)
+
+
+# the device's rule: a triangle with more than this many sources, or rows of
+# bins, to test is left to a workgroup, up to so many triangles
+MANY_SOURCES, MANY_ROWS, QUEUE = 512, 16, 1 << 18
+
+
+def _left(N, y, ys):
+    """How many triangles that rule leaves: the sources of the bins (as many as
+    the finite sources, over their extent) under the triangle's bounding box
+    and a bin around it; a triangle with a non-finite corner tests them all."""
+    if len(ys) <= MANY_SOURCES:
+        return 0
+    fin = ys[np.isfinite(ys).all(1)]
+    G = int(np.ceil(np.sqrt(len(fin))))
+    lo = fin.min(0)
+    w = G / np.ptp(fin, axis=0).max()
+    at = np.clip(np.floor((fin - lo) * w), 0, G - 1).astype(int)
+    cnt = np.zeros((G + 1, G + 1), np.int64)
+    np.add.at(cnt, (at[:, 1] + 1, at[:, 0] + 1), 1)
+    cnt = cnt.cumsum(0).cumsum(1)
+    k = (np.arange(N - 1)[:, None] * N + np.arange(N - 1)).ravel()
+    left = 0
+    for third in (k + 1, k + N):
+        t = np.stack([y[k], y[k + N + 1], y[third]], 1)
+        ok = np.isfinite(t).all((1, 2))
+        left += int((~ok).sum())
+        f0, f1 = (t[ok].min(1) - lo) * w, (t[ok].max(1) - lo) * w
+        hit = ~((f1 < -1).any(1) | (f0 > G).any(1))
+        b0 = np.maximum(np.floor(f0[hit]) - 1, 0).astype(int)
+        b1 = np.minimum(np.floor(f1[hit]) + 1, G - 1).astype(int)
+        n = (cnt[b1[:, 1] + 1, b1[:, 0] + 1] - cnt[b0[:, 1], b1[:, 0] + 1]
+             - cnt[b1[:, 1] + 1, b0[:, 0]] + cnt[b0[:, 1], b0[:, 0]])
+        left += int(((n > MANY_SOURCES) | (b1[:, 1] - b0[:, 1] >= MANY_ROWS)).sum())
+    return left
+
+
+def _load(ctx, N, y, A):
+    g = S.GridMap(S.Lens(ctx, 2.0), N, (0.0, 0.0), 1.0, shoot=False)
+    ctx.h2d(g.y_dev, np.ascontiguousarray(y))
+    ctx.h2d(g.A_dev, np.ascontiguousarray(A))
+    return g
+
+
+def _point_mass(N):
+    """y and A of a grid over a softened point mass: the cells beside it are
+    mapped over much of the source plane."""
+    x = O.gridmap_positions(N, (0.0, 0.0), 1.0)
+    r2 = (x ** 2).sum(1) + 1e-6
+    y = x - 0.04 * x / r2[:, None]
+    return x, y, np.random.default_rng(N).normal(size=(N * N, 4))
+
+
+@pytest.mark.parametrize("n", [513, 3000])
+@pytest.mark.parametrize("crowded", [False, True])
+def test_images_of_cells_over_many_sources(ctx, n, crowded):
+    """Cells by a point mass over evenly spread sources, and over a cluster of
+    them in one bin beside a few far ones: left to workgroups."""
+    N = 100
+    x, y, A = _point_mass(N)
+    rng = np.random.default_rng(n)
+    ys = (rng.random((n, 2)) - 0.5) * 2.0
+    if crowded:
+        ys[9:] = 0.1 + 1e-4 * rng.normal(size=(n - 9, 2))
+    assert _left(N, y, ys) > 0
+    g = _load(ctx, N, y, A)
+    assert _check(g, x, y, A, ys, 64).max() >= 2
+    g.close()
+
+
+def test_images_of_triangles_without_finite_corners(ctx):
+    """Infinite and NaN corners over more than 512 sources, one of them not
+    finite: every pair is tested, by workgroups."""
+    N, n = 64, 700
+    x, y, A = _point_mass(N)
+    y[[5, 900]] = np.nan
+    y[2000, 0] = np.inf
+    y[3000, 1] = -np.inf
+    ys = (np.random.default_rng(1).random((n, 2)) - 0.5) * 2.0
+    ys[7, 0] = np.inf
+    assert _left(N, y, ys) >= 20
+    g = _load(ctx, N, y, A)
+    _check(g, x, y, A, ys, 4096)
+    g.close()
+
+
+def test_images_of_more_triangles_than_the_queue_holds(ctx):
+    """Every triangle spans a cluster of sources, few contain it: the triangles
+    beyond the queue are tested where they are found."""
+    N, n = 400, 600
+    rng = np.random.default_rng(2)
+    i, j = np.meshgrid(np.arange(N), np.arange(N))
+    u = np.where((i + j) % 2 == 0, -1.0, 1.0).ravel()
+    y = np.stack([u, u], 1) + 0.01 * rng.normal(size=(N * N, 2))
+    y[rng.integers(0, N * N, 7)] = (0.8, -0.8)
+    y[rng.integers(N * (N - 20), N * N, 7)] = (0.8, -0.8)   # among the last cells
+    ys = np.array([0.4, -0.4]) + 0.05 * rng.normal(size=(n, 2))
+    assert _left(N, y, ys) > QUEUE + 10000
+    A = rng.normal(size=(N * N, 4))
+    x = O.gridmap_positions(N, (0.0, 0.0), 1.0)
+    g = _load(ctx, N, y, A)
+    assert _check(g, x, y, A, ys, 128).min() >= 40
+    g.close()
