@@ -156,3 +156,17 @@ def test_server_counts_the_rays_of_its_lists(ctx, field):
     srv.close()
     assert all(_same(ref, y, A) for y, A, _ in out)
     assert iterations * 32768 >= lists * planes * (n // 8)
+
+
+@pytest.mark.parametrize("N", [65, 129, 257])
+@pytest.mark.parametrize("precision", [S.SLSIM_FP64, S.SLSIM_FP32C])
+def test_rectangular_grid_is_the_grid_to_the_bit(field, N, precision):
+    """A rectangular GridMap's points go as a list.  Over a power of two of
+    radians with 2^k + 1 points a side they are the square GridMap's to the bit,
+    and so are its results."""
+    lens, _ = field
+    rg = 2.0 ** -10
+    a = S.GridMap.rect(lens, N, (0.0, 0.0), rg, rg, precision)
+    b = S.GridMap(lens, N, (0.0, 0.0), rg, precision)
+    assert np.array_equal(a.positions(), b.positions())
+    assert _same((a.y(), a.A()), b.y(), b.A())
