@@ -1392,12 +1392,12 @@ void k_plane_step_nfw(const StepJob* __restrict__ jobs, const WorkItem* __restri
 }
 
 // ------------------------------------------------------- lone-ray FP64 walk
-// One plane step of one ray per wavefront, for lists of few or scattered
-// rays, where a bundle walk would leave lanes idle and wait on one
-// wavefront's serial traversal.  The result is the bundle walk's to the bit:
-// the cells, the opening test and the terms are the same (include/quadTree.h:
-// 990-1128, the functions above), and the sums take the terms in the same
-// order, depth first, a popped entry's children last to first.
+// One plane step of one ray per block, for lists of few or scattered rays,
+// where a bundle walk would leave lanes idle and wait on one wavefront's serial
+// traversal.  The result is the bundle walk's to the bit: the cells, the opening
+// test and the terms are the same (include/quadTree.h:990-1128, the functions
+// above), and the sums take the terms in the same order, depth first, a popped
+// entry's children last to first.
 //
 // Two passes over a tree.  The first opens cells breadth first, sixteen
 // entries (64 children, a lane each) at a time, lists the opened cells in LDS
@@ -1413,16 +1413,18 @@ void k_plane_step_nfw(const StepJob* __restrict__ jobs, const WorkItem* __restri
 // entry's children are evaluated by themselves, and the opened ones' subtrees
 // go on a stack (a small opening angle; nothing is then too large).
 //
-// What bounds it is the latency of one wavefront's steps.  Of 364,000 cycles a
-// ray on the 65,536-particle halo (880 cells opened, 6,100 terms in 121
-// windows) the opening takes 54,000, the places 19,000, the cells' terms
+// What bounds it is the latency of a wavefront's steps.  Alone, a ray on the
+// 65,536-particle halo (880 cells opened, 6,100 terms in 121 windows) takes
+// 364,000 cycles: the opening 54,000, the places 19,000, the cells' terms
 // 55,000, the lists and particle loads 66,000, the particles' terms and the
 // writes to LDS 107,000 and the sums 62,000 (286,000 without the reads ahead
 // and with bank conflicts).  11 KB of LDS let 14 rays share a CU; a cap of 128
-// registers for a fourth wavefront a SIMD spilled and gained nothing.  40 rays
-// of that halo take 0.31 ms (4.0 ms by bundles; 0.13 ms with the terms summed
-// by lane, in no fixed order), 3,001 rays through four planes of 200,000
-// 1.41 ms (30 and 0.93 ms).
+// registers for a fourth wavefront a SIMD spilled and gained nothing.  While the
+// chip has room, four wavefronts share a ray: three make the terms of every
+// third batch, the first adds them: 187,000 cycles (eight wavefronts: the same).
+// 40 rays of that halo take 0.21 ms a call (4.0 ms by bundles; 0.13 ms with the
+// terms summed by lane, in no fixed order), 3,001 rays through four planes of
+// 200,000 1.4 ms (30 and 0.9 ms).
 namespace {
 
 constexpr int kLoneCells = 1024;   // opened cells listed at a time
@@ -1441,16 +1443,24 @@ constexpr int kFacKA = 6 * kWave + 22, kFacKB = 7 * kWave + 30, kLoneFactors = 8
 static_assert(kFacXA % 8 == 0 && kFacG0 % 8 == 2 && kFacG1 % 8 == 4 && kFacKA % 8 == 6, "banks");
 static_assert(kFacX0 % 8 == 0 && kFacX1 % 8 == 2 && kFacGB % 8 == 4 && kFacKB % 8 == 6, "banks");
 
+// NW wavefronts a ray: one does all, or the first adds the terms that the others
+// make, each in windows of its own.
+template <int NW>
 struct LoneShared {
+  static constexpr int kMakers = NW == 1 ? 1 : NW - 1, kWindows = NW == 1 ? 1 : 2;
   int32_t entry[kLoneCells];       // opened cells: first child | children << 28, breadth first
   uint16_t kids[kLoneCells];       // index of the first opened child | their number << 13;
                                    // then the depth-first order
   union {
     uint16_t size[kLoneCells];     // opened cells of the subtree; then the place
-    alignas(16) double factor[kLoneFactors];   // of a window's 64 terms
+    alignas(16) double factor[kMakers][kWindows][kLoneFactors];
   };
   int32_t stack[kStackDepth];
-  uint8_t own[kWave];
+  uint8_t own[kMakers][kWave];
+  int32_t opened[2][NW];           // cells opened by each wavefront in a step
+  // NW > 1: windows made and added up since the pass began, and each window's
+  // terms, negative for the last of its batch
+  int32_t made[kMakers], added[kMakers], terms[kMakers][kWindows];
 };
 
 template <int CTRL, int ROWS>
@@ -1487,19 +1497,21 @@ __device__ inline int lanes_before(uint64_t m) {
 // depth-first order in s.kids; returns their number, or -1 when they are more
 // than the list holds (then s.entry[1] on are top's opened children, s.kids[0]
 // their number << 13).
+template <int NW>
 __device__ int lone_open(const NodeD* __restrict__ nodes, int32_t top, double rx, double ry,
-                         LoneShared& s) {
+                         LoneShared<NW>& s) {
 #pragma clang fp contract(off)
-  const int lane = lane_id();
-  if (lane == 0) s.entry[0] = top;
+  const int lane = lane_id(), tid = (int)threadIdx.x, w = NW == 1 ? 0 : uni(tid >> 6);
+  if (tid == 0) s.entry[0] = top;
   __syncthreads();
-  int lo = 0, hi = 1, n = 1, nlev = 0;
+  int lo = 0, hi = 1, n = 1, nlev = 0, step = 0;
   int lev = 0;   // lane l: where level l starts
   constexpr int kStep = 2;   // loads of sixteen entries' children in flight
   while (lo < hi) {
     if (lane == nlev) lev = lo;
     ++nlev;
-    for (int b = lo; b < hi; b += 16 * kStep) {
+    for (int b0 = lo; b0 < hi; b0 += 16 * kStep * NW) {
+      const int b = b0 + 16 * kStep * w;
       int32_t opened[kStep];
       bool open[kStep];
 #pragma unroll
@@ -1515,21 +1527,38 @@ __device__ int lone_open(const NodeD* __restrict__ nodes, int32_t top, double rx
           opened[u] = nd.child | (nd.cmask << 28);
         }
       }
+uint64_t m[kStep];
+      int mine = 0;
 #pragma unroll
       for (int u = 0; u < kStep; ++u) {
-        const int i = b + 16 * u + (lane >> 2);
-        const uint64_t m = ballot(open[u]);
-        const int c = uni(__builtin_popcountll(m));
-        const int at = n + lanes_before(m);
-        if ((lane & 3) == 0 && i < hi)
-          s.kids[i] = (uint16_t)(at | (__builtin_popcountll((m >> lane) & 0xf) << 13));
-        if (n + c > kLoneCells) {
-          __syncthreads();
-          return -1;
-        }
-        if (open[u]) s.entry[at] = opened[u];
-        n += c;
+        m[u] = ballot(open[u]);
+        mine += uni(__builtin_popcountll(m[u]));
       }
+      int at = n, all = mine;
+      if (NW > 1) {
+        if (lane == 0) s.opened[step & 1][w] = mine;
+        __syncthreads();
+        all = 0;
+        for (int v = 0; v < NW; ++v) {
+          if (v < w) at += s.opened[step & 1][v];
+          all += s.opened[step & 1][v];
+        }
+        all = uni(all);
+        ++step;
+      }
+#pragma unroll
+      for (int u = 0; u < kStep; ++u) {
+        const int i = b + 16 * u + (lane >> 2), to = at + lanes_before(m[u]);
+        if ((lane & 3) == 0 && i < hi)
+          s.kids[i] = (uint16_t)(to | (__builtin_popcountll((m[u] >> lane) & 0xf) << 13));
+        if (open[u] && n + all <= kLoneCells) s.entry[to] = opened[u];
+        at += uni(__builtin_popcountll(m[u]));
+      }
+      if (n + all > kLoneCells) {
+        __syncthreads();
+        return -1;
+      }
+      n += all;
     }
     __syncthreads();
     lo = hi;
@@ -1538,7 +1567,7 @@ __device__ int lone_open(const NodeD* __restrict__ nodes, int32_t top, double rx
   for (int l = nlev - 1; l >= 0; --l) {
     const int a = __builtin_amdgcn_readlane(lev, l);
     const int e = l + 1 < nlev ? __builtin_amdgcn_readlane(lev, l + 1) : n;
-    for (int i = a + lane; i < e; i += kWave) {
+    for (int i = a + tid; i < e; i += NW * kWave) {
       const int kids = s.kids[i], f = kids & 8191, c = kids >> 13;
       int z[4];
 #pragma unroll
@@ -1550,11 +1579,11 @@ __device__ int lone_open(const NodeD* __restrict__ nodes, int32_t top, double rx
     }
     __syncthreads();
   }
-  if (lane == 0) s.size[0] = 0;
+  if (tid == 0) s.size[0] = 0;
   __syncthreads();
   for (int l = 0; l < nlev - 1; ++l) {
     const int a = __builtin_amdgcn_readlane(lev, l), e = __builtin_amdgcn_readlane(lev, l + 1);
-    for (int i = a + lane; i < e; i += kWave) {
+    for (int i = a + tid; i < e; i += NW * kWave) {
       const int kids = s.kids[i], f = kids & 8191, c = kids >> 13;
       int at = s.size[i] + 1, z[4];
 #pragma unroll
@@ -1567,7 +1596,7 @@ __device__ int lone_open(const NodeD* __restrict__ nodes, int32_t top, double rx
     }
     __syncthreads();
   }
-  for (int i = lane; i < n; i += kWave) s.kids[s.size[i]] = (uint16_t)i;
+  for (int i = tid; i < n; i += NW * kWave) s.kids[s.size[i]] = (uint16_t)i;
   __syncthreads();
   return n;
 }
@@ -1578,15 +1607,15 @@ constexpr int kLaneAx = 0, kLaneAy = 1, kLaneG0 = 4, kLaneG1 = 20, kLaneK = 8;
 
 // Adds a window's n terms to the sums, in order, four a step.
 // All is read ahead; volatile, or the compiler moves the reads to their uses.
-__device__ inline double lone_add(int n, double acc, const LoneShared& s) {
+__device__ inline double lone_add(int n, double acc, const double* factor) {
   typedef double d2 __attribute__((ext_vector_type(2)));
   const int lane = lane_id(), block = (lane >> 2) & 3, ij = lane & 1, k = (lane >> 4) << 3;
   const int a = (block == 1 ? (ij ? kFacG1 : kFacG0) : (block == 2 ? kFacKA : kFacXA)) + k;
   const int b = (block == 1 ? kFacGB : (block == 2 ? kFacKB : (ij ? kFacX1 : kFacX0))) + k;
   d2 va[2][4], vb[2][4];
   auto load = [&](int h) {
-    const lds_ptr<d2> pa = (lds_ptr<d2>)(s.factor + a + kPass * h);
-    const lds_ptr<d2> pb = (lds_ptr<d2>)(s.factor + b + kPass * h);
+    const lds_ptr<d2> pa = (lds_ptr<d2>)(factor + a + kPass * h);
+    const lds_ptr<d2> pb = (lds_ptr<d2>)(factor + b + kPass * h);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       va[h][u] = pa[u];
@@ -1608,12 +1637,33 @@ __device__ inline double lone_add(int n, double acc, const LoneShared& s) {
   return acc;
 }
 
-// The children of the n listed cells, in order, 64 terms a window.  The next
-// window's particles are loaded while a window's terms are added up, the next
-// cells a batch ahead.
-__device__ double lone_eval64(const TreeDesc& t, int n, double rx, double ry, double acc,
-                              LoneShared& s) {
+// Orders a wavefront's own LDS accesses, between its lanes.
+__device__ inline void lone_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Waits until another wavefront of the block has counted *p up to v.
+__device__ inline void lone_wait(const int32_t* p, int v) {
+  while (__hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < v)
+    __builtin_amdgcn_s_sleep(1);
+}
+__device__ inline void lone_count(int32_t* p, int v) {
+  if (lane_id() == 0) __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// The terms of the children of the n listed cells, in order, 64 a window, by
+// wavefront `maker`, which takes every kMakers-th batch of sixteen cells.  A lone
+// wavefront adds a window up itself, while the next window's particles are on
+// their way; else a window is handed to the adding wavefront (lone_sum), which
+// takes the batches in order: it only ever waits for the next window of one
+// maker, and that maker only for a window that it has taken, so neither waits
+// for good.
+template <int NW>
+__device__ double lone_make64(const TreeDesc& t, int n, double rx, double ry, double acc,
+                              int maker, LoneShared<NW>& s) {
 #pragma clang fp contract(off)
+  constexpr int kMakers = LoneShared<NW>::kMakers, kWindows = LoneShared<NW>::kWindows;
   const int lane = lane_id(), child = 3 - (lane & 3);
   const NodeD* __restrict__ nodes = t.nodesD;
   const PartD* __restrict__ parts = t.partsD;
@@ -1628,8 +1678,9 @@ __device__ double lone_eval64(const TreeDesc& t, int n, double rx, double ry, do
     there = (e >> (28 + child)) & 1;
     if (there) nd = nodes[(e & 0x0fffffff) + child];
   };
-  load(0);
-  bool kappa_zero = false;   // kappa's factors are zeros
+  load(16 * maker);
+  int kappa_zero = 0;   // windows whose kappa factors are zeros (bits)
+  int windows = 0;
   // A lane's child of the batch's sixteen cells adds a far cell's term (far),
   // or a list of particles: a leaf's `cnt`, then their corrections when it is
   // near (kind 1), or an internal cell's big particles' corrections (kind 2).
@@ -1642,11 +1693,14 @@ __device__ double lone_eval64(const TreeDesc& t, int n, double rx, double ry, do
   // cell).
   int o_kind = 0, o_cnt = 0, q = 0, nw = 0;
   PartD pt{};
-  int total = 0, w0 = 0, k0 = -16;   // the batch's terms, the window, the batch
+  // the batch's terms, the window, the batch
+  int total = 0, w0 = 0, k0 = 16 * (maker - kMakers);
   for (bool have = false;; have = true) {
     bool kappa = sheet;
-    const int nw_now = nw;
+    const int nw_now = nw, slot = windows % kWindows;
+    double* const factor = s.factor[maker][slot];
     if (have) {
+      if (NW > 1) lone_wait(&s.added[maker], windows - kWindows + 1);
       bool spline = false;
       double ka = 0, kb = 0;
       const bool mine = lists && lane < nw && o_kind != 0;
@@ -1688,47 +1742,57 @@ __device__ double lone_eval64(const TreeDesc& t, int n, double rx, double ry, do
             spline = true;
           }
         }
-        s.factor[kFacXA + at] = xa;
-        s.factor[kFacX0 + at] = xb0;
-        s.factor[kFacX1 + at] = xb1;
-        s.factor[kFacG0 + at] = ga0;
-        s.factor[kFacG1 + at] = ga1;
-        s.factor[kFacGB + at] = gb;
+        factor[kFacXA + at] = xa;
+        factor[kFacX0 + at] = xb0;
+        factor[kFacX1 + at] = xb1;
+        factor[kFacG0 + at] = ga0;
+        factor[kFacG1 + at] = ga1;
+        factor[kFacGB + at] = gb;
       }
       kappa = kappa || ballot(spline) != 0;
       const int g = pre - w0, ag = factor_at(g);
       const bool far_here = far && g >= 0 && g < kWave;
       if (far_here) {
-        s.factor[kFacXA + ag] = 1.0;
-        s.factor[kFacX0 + ag] = f.ax;
-        s.factor[kFacX1 + ag] = f.ay;
-        s.factor[kFacG0 + ag] = f.h;
-        s.factor[kFacG1 + ag] = f.xy;
-        s.factor[kFacGB + ag] = f.w;
+        factor[kFacXA + ag] = 1.0;
+        factor[kFacX0 + ag] = f.ax;
+        factor[kFacX1 + ag] = f.ay;
+        factor[kFacG0 + ag] = f.h;
+        factor[kFacG1 + ag] = f.xy;
+        factor[kFacGB + ag] = f.w;
       }
       const bool fill = lane >= nw && lane < ((nw + kPass - 1) & ~(kPass - 1));
       if (fill)
-        s.factor[kFacXA + at] = s.factor[kFacX0 + at] = s.factor[kFacX1 + at] =
-            s.factor[kFacG0 + at] = s.factor[kFacG1 + at] = s.factor[kFacGB + at] = 0.0;
+        factor[kFacXA + at] = factor[kFacX0 + at] = factor[kFacX1 + at] =
+            factor[kFacG0 + at] = factor[kFacG1 + at] = factor[kFacGB + at] = 0.0;
       if (kappa) {
         if (mine || fill) {
-          s.factor[kFacKA + at] = ka;
-          s.factor[kFacKB + at] = kb;
+          factor[kFacKA + at] = ka;
+          factor[kFacKB + at] = kb;
         }
         if (far_here) {
-          s.factor[kFacKA + ag] = sheet ? -(ia * mass) : 0.0;
-          s.factor[kFacKB + ag] = sheet ? 1.0 : 0.0;
+          factor[kFacKA + ag] = sheet ? -(ia * mass) : 0.0;
+          factor[kFacKB + ag] = sheet ? 1.0 : 0.0;
         }
-        kappa_zero = false;
-      } else if (!kappa_zero) {
-        s.factor[kFacKA + lane] = s.factor[kFacKB + lane] = 0.0;
-        kappa_zero = true;
+        kappa_zero &= ~(1 << slot);
+      } else if (!((kappa_zero >> slot) & 1)) {
+        factor[kFacKA + lane] = factor[kFacKB + lane] = 0.0;
+        kappa_zero |= 1 << slot;
       }
-      __syncthreads();
+      if (NW == 1) {
+        __syncthreads();
+      } else {
+        if (lane == 0) s.terms[maker][slot] = w0 + kWave >= total ? -1 - nw : nw;
+        lone_count(&s.made[maker], ++windows);
+      }
     }
     // on to the next window
     for (w0 += kWave; w0 >= total && k0 < n; w0 = 0) {
-      k0 += 16;
+      if (NW > 1 && total == 0 && k0 >= 0) {   // a batch without a term
+        lone_wait(&s.added[maker], windows - kWindows + 1);
+        if (lane == 0) s.terms[maker][windows % kWindows] = -1;
+        lone_count(&s.made[maker], ++windows);
+      }
+      k0 += 16 * kMakers;
       total = 0;
       if (k0 >= n) break;
       far = false;
@@ -1755,7 +1819,7 @@ __device__ double lone_eval64(const TreeDesc& t, int n, double rx, double ry, do
           }
         }
       }
-      load(k0 + 16);
+      load(k0 + 16 * kMakers);
       pre = wave_scan(terms) - terms;
       total = uni(__builtin_amdgcn_readlane(pre + terms, 63));
       lists = ballot(kind != 0 && terms > 0) != 0;
@@ -1766,14 +1830,14 @@ __device__ double lone_eval64(const TreeDesc& t, int n, double rx, double ry, do
       if (lists) {
         // the child that the window's lane-th term belongs to: the last that
         // starts at or before it
-        s.own[lane] = 0;
-        __syncthreads();
+        s.own[maker][lane] = 0;
+        lone_fence();
         const int behind = __shfl_down(pre, 1, kWave);
         const int end = lane < 63 ? behind : total;
         if (end > pre && pre < w0 + kWave && end > w0)
-          s.own[pre > w0 ? pre - w0 : 0] = (uint8_t)(lane + 1);
-        __syncthreads();
-        const int o = wave_scan_max(s.own[lane]) - 1;
+          s.own[maker][pre > w0 ? pre - w0 : 0] = (uint8_t)(lane + 1);
+        lone_fence();
+        const int o = wave_scan_max(s.own[maker][lane]) - 1;
         o_kind = __shfl(kind, o, kWave);
         o_cnt = __shfl(cnt, o, kWave);
         const int o_start = __shfl(start, o, kWave);
@@ -1782,34 +1846,62 @@ __device__ double lone_eval64(const TreeDesc& t, int n, double rx, double ry, do
           pt = (o_kind == 2 ? bigs : parts)[o_start + (q < o_cnt ? q : q - o_cnt)];
       }
     }
-    if (have) {
-      acc = lone_add(nw_now, acc, s);
+    if (NW == 1 && have) {
+      acc = lone_add(nw_now, acc, factor);
       __syncthreads();
     }
     if (!more) return acc;
   }
 }
 
-__device__ double lone_walk64(const TreeDesc& t, double rx, double ry, LoneShared& s) {
-  const int lane = lane_id();
+// Adds up the makers' windows of the n listed cells, batch by batch.
+template <int NW>
+__device__ double lone_sum(int n, double acc, LoneShared<NW>& s) {
+  constexpr int kMakers = LoneShared<NW>::kMakers, kWindows = LoneShared<NW>::kWindows;
+  int taken = 0;   // lane m: windows taken from maker m
+  for (int k0 = 0, maker = 0; k0 < n; k0 += 16, maker = maker + 1 < kMakers ? maker + 1 : 0) {
+    for (bool last = false; !last;) {
+      const int at = __builtin_amdgcn_readlane(taken, maker), slot = at % kWindows;
+      lone_wait(&s.made[maker], at + 1);
+      const int v = uni(s.terms[maker][slot]), nw = v < 0 ? -1 - v : v;
+      last = v < 0;
+      if (nw > 0) acc = lone_add(nw, acc, s.factor[maker][slot]);
+      lone_count(&s.added[maker], at + 1);
+      if (lane_id() == maker) ++taken;
+    }
+  }
+  return acc;
+}
+
+template <int NW>
+__device__ double lone_walk64(const TreeDesc& t, double rx, double ry, LoneShared<NW>& s) {
+  const int tid = (int)threadIdx.x, w = NW == 1 ? 0 : uni(tid >> 6);
   double acc = 0.0;
-  if (lane == 0) s.stack[0] = 1 << 28;   // the root as the only child of a virtual cell
+  if (tid == 0) s.stack[0] = 1 << 28;   // the root as the only child of a virtual cell
   int sp = 1;
   __syncthreads();
   while (sp > 0) {
     const int32_t top = uni(s.stack[--sp]);
-    int n = lone_open(t.nodesD, top, rx, ry, s);
+    int n = lone_open<NW>(t.nodesD, top, rx, ry, s);
     if (n < 0) {
       // top by itself, then its opened children's subtrees, the first on top
       const int c = uni(s.kids[0]) >> 13;
-      if (lane < c) s.stack[sp + c - 1 - lane] = s.entry[1 + lane];
+      if (tid < c) s.stack[sp + c - 1 - tid] = s.entry[1 + tid];
       sp += c;
       __syncthreads();
-      if (lane == 0) s.kids[0] = 0;
-      __syncthreads();
+      if (tid == 0) s.kids[0] = 0;
       n = 1;
     }
-    acc = lone_eval64(t, n, rx, ry, acc, s);
+    if (NW == 1) {
+      __syncthreads();
+      acc = lone_make64<NW>(t, n, rx, ry, acc, 0, s);
+    } else {
+      if (tid < LoneShared<NW>::kMakers) s.made[tid] = s.added[tid] = 0;
+      __syncthreads();
+      if (w == 0) acc = lone_sum<NW>(n, acc, s);
+      else lone_make64<NW>(t, n, rx, ry, 0.0, w - 1, s);
+      __syncthreads();
+    }
   }
   return acc;
 }
@@ -1817,12 +1909,13 @@ __device__ double lone_walk64(const TreeDesc& t, double rx, double ry, LoneShare
 }  // namespace
 
 // A plane step of each listed ray (items == null: rays 0 .. nitems - 1 of
-// jobs[0]; slot = ray, dense state), one wavefront per ray; planes of particle
-// trees only.
-__global__ __launch_bounds__(kWave) void k_plane_step_lone(const StepJob* __restrict__ jobs,
+// jobs[0]; slot = ray, dense state), one block of NW wavefronts per ray; planes
+// of particle trees only.
+template <int NW>
+__global__ __launch_bounds__(NW* kWave) void k_plane_step_lone(const StepJob* __restrict__ jobs,
                                                           const WorkItem* __restrict__ items,
                                                           uint32_t nitems) {
-  __shared__ LoneShared s;
+  __shared__ LoneShared<NW> s;
   const uint32_t r = xcd_block(blockIdx.x, gridDim.x);
   if (r >= nitems) return;
   WorkItem it{0u, r};
@@ -1839,7 +1932,7 @@ __global__ __launch_bounds__(kWave) void k_plane_step_lone(const StepJob* __rest
   const int ntrees = uni(jb.ntrees);
   for (int h = 0; h < ntrees; ++h) {
     const TreeDesc t = as_const(jb.trees)[h];
-    tot += lone_walk64(t, rx, ry, s);
+    tot += lone_walk64<NW>(t, rx, ry, s);
   }
   const double alpha0 = __shfl(tot, kLaneAx, kWave), alpha1 = __shfl(tot, kLaneAy, kWave);
   const double gamma0 = __shfl(tot, kLaneG0, kWave), gamma1 = __shfl(tot, kLaneG1, kWave);
@@ -2303,7 +2396,11 @@ void launch_plane_steps_fused(int precision, unsigned nblocks, uint32_t nitems, 
 
 void launch_plane_step_lone(hipStream_t st, const StepJob* jobs, const WorkItem* items,
                             uint32_t nitems) {
-  if (nitems > 0) k_plane_step_lone<<<nitems, kWave, 0, st>>>(jobs, items, nitems);
+  if (nitems == 0) return;
+  if (nitems <= kLoneFewRays)
+    k_plane_step_lone<4><<<nitems, 4 * kWave, 0, st>>>(jobs, items, nitems);
+  else
+    k_plane_step_lone<1><<<nitems, kWave, 0, st>>>(jobs, items, nitems);
 }
 
 void launch_zero_u32(hipStream_t st, uint32_t* p, int n) {

@@ -237,6 +237,12 @@ constexpr int64_t kGuardLoneRays = 8192;
 //   two planes of 2^20, 300":         20,000 rays 4.34 / 4.50 and 4.02 / 20.2
 // (square grids of rays as lists are like the second of each).
 constexpr size_t kLoneRays64 = 20000;
+// A launch of up to this many lone rays gives each four wavefronts; 33 KB of LDS
+// let four rays share a CU then.  Wall us of a call with four / one, scattered
+// over the halo's field and over the planes of 2^20: 40 rays 207 / 289 and 400 /
+// 579, 1,024 rays 250 / 308 and 535 / 707, 1,500 rays 314 / 324 and 758 / 769,
+// 2,048 rays 384 / 345 and 842 / 774; clustered ones cross at 1,200 to 1,400.
+constexpr uint32_t kLoneFewRays = 1024;
 
 // FP32C lists are spread over up to this many wavefronts, one a SIMD, with as
 // few rays each as that takes: a wavefront walks the union of its rays' cells.
@@ -463,7 +469,7 @@ struct FlatLCDM;
 // that walk them)
 void launch_plane_step(int precision, bool count, uint32_t nitems, hipStream_t st,
                        const StepJob* jobs, const WorkItem* items, uint32_t* err, int halos);
-// a plane step of single rays, a wavefront each: item i is (job, slot);
+// a plane step of single rays, one or four wavefronts each: item i is (job, slot);
 // items == nullptr: slots 0 .. nitems-1 of job 0 (FP64, planes of particle
 // trees only)
 void launch_plane_step_lone(hipStream_t st, const StepJob* jobs, const WorkItem* items,

@@ -1,5 +1,6 @@
-"""Ray lists on the lone-ray FP64 walk: the sizes where its launch changes
-(the bundle walk beyond 20,000 rays), coarse leaves and big particles, against
+"""Ray lists at the sizes where their launch changes (FP64: the lone-ray walk
+with four wavefronts a ray up to 1,024, with one up to 20,000, bundles beyond;
+FP32C: 1 to 64 rays a bundle), on coarse leaves and with big particles, against
 the oracle and, to the bit, against the grid launch.
 
 Tolerance: the same algorithm in the same precision, sums in another order:
@@ -76,7 +77,7 @@ def _same(r, y, A):
     return np.array_equal(r[0], y) and np.array_equal(r[1], A)
 
 
-@pytest.mark.parametrize("N", [1, 6, 8, 45, 46, 90, 127, 141, 142, 222])
+@pytest.mark.parametrize("N", [1, 6, 8, 32, 33, 45, 46, 90, 127, 141, 142, 222])
 def test_list_is_its_gridmap_to_the_bit(ctx, field, N):
     """A ray's FP64 result does not depend on the rays beside it: the rays of
     a GridMap as a list in another order, as two lists, and as a served list
@@ -113,8 +114,9 @@ def test_trees_of_any_form_give_the_grid_bits(ctx, bucket, max_range, theta):
     for z, ia in ((0.5, 0.0), (0.5, 30.0), (1.0, 0.0)):
         lens.moveinMainHalo(S.LensHaloParticles(ctx, x, y, m, h, z, bucket=bucket, theta=theta,
                                                 inv_area=ia, max_range=max_range))
-    g = S.GridMap(lens, 30, (0.0, 0.0), W.grid_range(60.0), S.SLSIM_FP64)
-    assert _same(lens.rayshooterInternal(g.positions()), g.y(), g.A())
+    for N in (30, 40):                    # four wavefronts a ray, and one
+        g = S.GridMap(lens, N, (0.0, 0.0), W.grid_range(60.0), S.SLSIM_FP64)
+        assert _same(lens.rayshooterInternal(g.positions()), g.y(), g.A())
     lens.close()
 
 
