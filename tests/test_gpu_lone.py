@@ -100,7 +100,8 @@ def test_list_is_its_gridmap_to_the_bit(ctx, field, N):
 
 @pytest.mark.parametrize("bucket,max_range,theta", [(1, -1.0, 0.1), (20, -1.0, 0.1),
                                                     (700, -1.0, 0.1), (20, 0.02, 0.1),
-                                                    (5, -1.0, 0.004), (1, -1.0, 0.5)])
+                                                    (5, -1.0, 0.004), (1, -1.0, 0.004),
+                                                    (1, -1.0, 0.5)])
 def test_trees_of_any_form_give_the_grid_bits(ctx, bucket, max_range, theta):
     """As above on coarse leaves, big particles, a mass sheet and, at the
     smallest opening angle, more opened cells than the walk lists at a time."""
