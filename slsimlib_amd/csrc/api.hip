@@ -962,15 +962,6 @@ int shoot_array(slsim_lens L, size_t n, const double* x_dev, const double* zs_de
   if (guard_after && particle_planes(L)) {
     lanes = 1;
     while (lanes < kWave && (int64_t)n > lanes * kSparseWaves32) lanes *= 2;
-    // (the slots of sparse bundles, at most 8 MiB of state, are not worth a
-    // refused call where a context's budget is nearly spent)
-    size_t room;
-    {
-      std::lock_guard<std::mutex> g(c->mu);
-      room = c->budget - c->used;
-      for (const auto& a : c->cache) room += a.second;
-    }
-    if (room < 8 * kStateBytesPerSlot * kWave * (n / lanes + 1)) lanes = kWave;
   }
   if (lanes <= 0) lanes = kWave;
   if (lanes > kWave) return arg_error("bad rays per bundle");

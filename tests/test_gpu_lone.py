@@ -173,22 +173,3 @@ def test_rectangular_grid_is_the_grid_to_the_bit(field, N, precision):
     b = S.GridMap(lens, N, (0.0, 0.0), rg, precision)
     assert np.array_equal(a.positions(), b.positions())
     assert _same((a.y(), a.A()), b.y(), b.A())
-
-
-def test_fp32c_list_in_a_context_with_little_room():
-    """Short FP32C lists take sparse bundles, whose slots need more memory than
-    the list; where the context's budget has no room for them they take full
-    ones, with the same results."""
-    rng = np.random.default_rng(3)
-    x, y = 0.05 * rng.normal(size=(2, 4000))
-    m, h = np.full(4000, 1e9, np.float32), np.full(4000, 1e-4, np.float32)
-    pos = (rng.random((1000, 2)) - 0.5) * W.grid_range(60.0)
-    c = S.Context(0, hbm_budget=256 << 20)
-    lens = S.Lens(c, 2.0)
-    lens.moveinMainHalo(S.LensHaloParticles(c, x, y, m, h, 0.5))
-    free = lens.rayshooterInternal(pos, precision=S.SLSIM_FP32C)
-    used, budget = c.memory()
-    c.alloc(budget - used - (2 << 20))
-    assert _same(lens.rayshooterInternal(pos, precision=S.SLSIM_FP32C), *free)
-    lens.close()
-    c.close()
