@@ -227,12 +227,16 @@ typedef struct {
  * (FullRange/internal_rayshooter_multi.cpp:53-251; include/lens.h:913-1103).
  * Host buffers: x (2n, x0 x1 interleaved, radians), zs (n source redshifts or
  * NULL = lens source), y (2n out), A (4n out, row-major a0 a1 a2 a3).
- * Rays are Morton-ordered on the device so that each wavefront walks a
- * spatially coherent bundle; short SLSIM_FP64 lists take a wavefront per ray.
- * A ray's result does not depend on that, or on the rays beside it: it is to
- * the bit what a GridMap with that ray gives (SLSIM_FP32C: as long as the
- * guard, whose limits are relative to the call's rms deflection, decides
- * alike).  Results come back in input order.
+ * Large lists are Morton-ordered on the device so that each wavefront walks a
+ * spatially coherent bundle; short lists take a wavefront or more per ray.
+ * SLSIM_FP64: a ray's result does not depend on that, or on the rays beside it;
+ * it is to the bit what a GridMap with that ray gives.  SLSIM_FP32C: lists of
+ * more than 16,000 rays, and lists through analytic halos, give the SLSIM_FP32C
+ * GridMap's results to the bit (as long as the guard, whose limits are relative
+ * to the call's rms deflection, decides alike); shorter ones are shot in FP64
+ * and give the SLSIM_FP64 GridMap's, n_guarded 0, so a list of more rays, split
+ * or joined across that line, gives values that differ by the FP32 walk's error.
+ * Results come back in input order.
  */
 int slsim_shoot(slsim_lens lens, size_t n, const double* x, const double* zs, double* y,
                 double* A, int precision, slsim_shoot_stats* stats);

@@ -829,9 +829,11 @@ static bool particle_planes(const slsim_lens_s* L) {
   return true;
 }
 
-// Whether a list of n rays goes to the lone-ray walk.
+// Whether a list of n rays goes to the lone-ray FP64 walk (either precision:
+// its FP64 results need no guard).
 bool list_is_lone(const slsim_lens_s* L, size_t n, int precision) {
-  return precision == SLSIM_FP64 && n <= kLoneRays64 && particle_planes(L);
+  if (precision != SLSIM_FP64 && precision != SLSIM_FP32C) return false;
+  return n <= (precision == SLSIM_FP64 ? kLoneRays64 : kLoneRays32) && particle_planes(L);
 }
 
 void make_steps(const slsim_lens_s* L, const RayState& st, int64_t nslots, uint32_t* counters,
@@ -956,13 +958,10 @@ int shoot_array(slsim_lens L, size_t n, const double* x_dev, const double* zs_de
   // lanes < 0: the list's own rule; 0: the lone-ray FP64 walk where every
   // plane has particle trees only, else full bundles.  Lone rays are dense in
   // the state, in the list's order.
-  const bool guard_after = precision == SLSIM_FP32C && lanes < 0;
+  const bool guard_after = precision == SLSIM_FP32C && lanes < 0 && !list_is_lone(L, n, precision);
   const bool lone = lanes == 0 ? precision == SLSIM_FP64 && particle_planes(L)
                                : lanes < 0 && list_is_lone(L, n, precision);
-  if (guard_after && particle_planes(L)) {
-    lanes = 1;
-    while (lanes < kWave && (int64_t)n > lanes * kSparseWaves32) lanes *= 2;
-  }
+  if (lone) precision = SLSIM_FP64;
   if (lanes <= 0) lanes = kWave;
   if (lanes > kWave) return arg_error("bad rays per bundle");
   const int64_t nbundles = ((int64_t)n + lanes - 1) / lanes;
@@ -1022,7 +1021,6 @@ int shoot_array(slsim_lens L, size_t n, const double* x_dev, const double* zs_de
     m.x = x_dev;
     m.zs = zs_dev;
     m.n = (int64_t)n;
-    m.lanes = lanes;
     int32_t ng = 0;
     if ((rc = guard_refine(L, st, nslots, m, (int64_t)n, zs_dev, zs_uniform, y_dev, A_dev, s,
                            &ng)))

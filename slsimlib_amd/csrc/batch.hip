@@ -791,13 +791,13 @@ void slsim_server_s::loop() {
       rc = SLSIM_ERR_TOO_DEEP;
     // the precision form's guard of each finished request, as a lone shoot's
     for (Req* r : finished) {
-      if (rc || r->precision != SLSIM_FP32C || r->jmax <= 0) continue;
+      if (rc || r->precision != SLSIM_FP32C || r->jmax <= 0 || r->unit != kWave)
+        continue;
       GuardMap m{};
       if (r->nrays > 0) {
         m.x = r->xd;
         m.zs = r->zsd;
         m.n = r->nrays;
-        m.lanes = kWave;
       } else {
         m.N = r->N;
         m.tiles_x = r->tiles_x;

@@ -2114,7 +2114,7 @@ __global__ void k_finalize_array(RayState st, int64_t nslots, int64_t n,
 
 // ----------------------------------------------- precision-form guard
 // A call's slots: ray i and its image position.  Grid: the tiles of a
-// GridMap; array: sorted ray k, ray perm[k] of x.
+// GridMap; array: slot s < n holds ray perm[s] of x.
 __device__ inline bool slot_ray(const GuardMap& m, int64_t slot, int64_t* i, double* x0,
                                 double* x1) {
   if (m.x == nullptr) {
@@ -2122,9 +2122,8 @@ __device__ inline bool slot_ray(const GuardMap& m, int64_t slot, int64_t* i, dou
     grid_position(*i, m.N, m.c0, m.c1, m.range, x0, x1);
     return true;
   }
-  const int64_t k = array_ray_index(slot, m.lanes);
-  if (k < 0 || k >= m.n) return false;
-  *i = m.perm ? (int64_t)m.perm[k] : k;
+  if (slot >= m.n) return false;
+  *i = m.perm ? (int64_t)m.perm[slot] : slot;
   *x0 = m.x[2 * *i];
   *x1 = m.x[2 * *i + 1];
   return true;

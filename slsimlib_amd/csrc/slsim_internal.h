@@ -226,17 +226,23 @@ constexpr double kGuardSmallAlpha = 0.01;
 constexpr int64_t kGuardWaves = 8192;
 // up to this many re-shot rays: the lone-ray walk
 constexpr int64_t kGuardLoneRays = 8192;
-// FP64 lists of up to this many rays go to the lone-ray walk.  Its time grows
-// with the rays, the bundle walk's is its slowest wavefront's however few there
-// are.  Results are the same to the bit either way, so the line lies where the
+// Lists of up to this many rays go to the lone-ray walk.  Its time grows with
+// the rays, the bundle walk's is its slowest wavefront's however few there are.
+// FP64 results are the same to the bit either way, so the line lies where the
 // bundles catch up on the lists that suit them best, clustered ones.  Wall ms of
 // a call, lone / bundles, lists over 0.02 of the field and over all of it:
 //   65,536-particle halo, 30":        16,000 rays 1.97 / 2.26 and 1.41 / 3.71,
 //                                     20,000 rays 2.38 / 2.28 and 1.70 / 3.47
 //   two planes of 200,000, 300":      20,000 rays 2.76 / 3.16 and 2.62 / 10.5
 //   two planes of 2^20, 300":         20,000 rays 4.34 / 4.50 and 4.02 / 20.2
-// (square grids of rays as lists are like the second of each).
-constexpr size_t kLoneRays64 = 20000;
+// (square grids of rays as lists are like the second of each).  SLSIM_FP32C:
+// such lists are shot in FP64, which leaves nothing to guard: the FP32C walk
+// takes 1.8 to 3.9 ms for 40 rays of these fields even with a ray a bundle, the
+// lone walk 0.2 to 0.4.  Clustered ones break even with FP32C bundles at 19,000
+// to 22,000 rays as well, but the line lies lower there, because results change
+// at it: FP64 below, the FP32C GridMap's to the bit above, where lists as long as
+// a 128 x 128 grid's belong.
+constexpr size_t kLoneRays64 = 20000, kLoneRays32 = 16000;
 // A launch of up to this many lone rays gives each four wavefronts; 33 KB of LDS
 // let four rays share a CU then.  Wall us of a call with four / one, scattered
 // over the halo's field and over the planes of 2^20: 40 rays 207 / 289 and 400 /
@@ -244,20 +250,12 @@ constexpr size_t kLoneRays64 = 20000;
 // 2,048 rays 384 / 345 and 842 / 774; clustered ones cross at 1,200 to 1,400.
 constexpr uint32_t kLoneFewRays = 1024;
 
-// FP32C lists are spread over up to this many wavefronts, one a SIMD, with as
-// few rays each as that takes: a wavefront walks the union of its rays' cells.
-// Wall ms of a call, spread / 64 rays a bundle, rays over the fields above: 40
-// rays 1.8 / 6.3, 2.8 / 26, 3.9 / 59; 3,000 rays 2.5 / 3.4, 5.3 / 10, 7.9 / 26;
-// clustered lists the same either way (with 2,048 wavefronts 8,000 of them took
-// 2.5 / 2.1, 2.9 / 2.8, 4.3 / 4.0).
-constexpr int64_t kSparseWaves32 = 1024;
-
 // A call's slots for the guard kernels: x == null: the tiles of an N x N
-// GridMap; else sorted ray k, `lanes` of them a bundle, is ray perm[k] (perm ==
-// null: ray k) of x, with per-ray source redshifts zs (or null).
+// GridMap; else slot s < n holds ray perm[s] (perm == null: ray s) of x,
+// with per-ray source redshifts zs (or null).
 struct GuardMap {
   int64_t N, tiles_x;
-  int32_t tw, lanes;
+  int32_t tw, pad;
   double c0, c1, range;
   const uint32_t* perm;
   const double* x;

@@ -93,7 +93,8 @@ def test_precision_form_fp64_matches_oracle(c3_small):
 def test_precision_form_guard_same_for_ray_lists(c3_small):
     """The guard's decisions depend on a ray alone (and the call's rms), so
     the rays of a GridMap shot as a list in another order give the same
-    results bit for bit."""
+    results bit for bit (a list of more than 16,000 rays: shorter ones are
+    shot in FP64, tests/test_gpu_lone.py)."""
     N, rg = 128, W.grid_range(300.0)
     g32 = S.GridMap(c3_small["lens"], N, (0.0, 0.0), rg, S.SLSIM_FP32C)
     x = g32.positions()

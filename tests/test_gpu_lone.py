@@ -1,7 +1,7 @@
 """Ray lists at the sizes where their launch changes (FP64: the lone-ray walk
 with four wavefronts a ray up to 1,024, with one up to 20,000, bundles beyond;
-FP32C: 1 to 64 rays a bundle), on coarse leaves and with big particles, against
-the oracle and, to the bit, against the grid launch.
+FP32C: shot in FP64 up to 16,000), on coarse leaves and with big particles,
+against the oracle and, to the bit, against the grid launch.
 
 Tolerance: the same algorithm in the same precision, sums in another order:
 relative |d alpha| <= 1e-9, |d A| <= 1e-8 (the bounds of the FP64 walk's tests).
@@ -15,7 +15,7 @@ from slsimlib_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
 
-LIMIT64, SPARSE = 20000, 1024   # rays: to the lone walk; FP32C bundles not yet full, per ray of each
+LIMIT64, LIMIT32, FOUR_WAVES = 20000, 16000, 1024
 
 
 def _check(lens, L, x, y, A, zs=None):
@@ -37,8 +37,8 @@ def field(ctx):
     return lens, L
 
 
-@pytest.mark.parametrize("n", [1, 63, 64, 65, SPARSE, SPARSE + 1, 16000, 16001, LIMIT64,
-                               LIMIT64 + 1, 32 * SPARSE, 32 * SPARSE + 1, 49152, 49153])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, FOUR_WAVES, FOUR_WAVES + 1, 2048, 2049, LIMIT32,
+                               LIMIT32 + 1, LIMIT64, LIMIT64 + 1, 49152, 49153])
 def test_list_sizes_match_oracle(field, n):
     lens, L = field
     rng = np.random.default_rng(n)
@@ -46,8 +46,11 @@ def test_list_sizes_match_oracle(field, n):
     zs = rng.uniform(0.05, 4.0, n) if n % 2 else None
     y, A = lens.rayshooterInternal(x, zs)
     _check(lens, L, x, y, A, zs)
+    st = {}
+    y32, A32 = lens.rayshooterInternal(x, zs, S.SLSIM_FP32C, stats=st)
+    if n <= LIMIT32:                      # FP64 results: nothing to guard
+        assert np.array_equal(y32, y) and np.array_equal(A32, A) and st["n_guarded"] == 0
     # the precision form within its bound of the FP64 path at every ray
-    y32, A32 = lens.rayshooterInternal(x, zs, S.SLSIM_FP32C)
     a = np.linalg.norm(x - y, axis=1)
     scale = np.maximum(a, 1e-3 * np.sqrt(np.mean(a ** 2)))
     assert (np.linalg.norm(y32 - y, axis=1) <= 1e-5 * scale).all()
@@ -121,24 +124,33 @@ def test_trees_of_any_form_give_the_grid_bits(ctx, bucket, max_range, theta):
     lens.close()
 
 
-@pytest.mark.parametrize("N", [2, 8, 31, 32, 33, 45, 46, 64, 126, 127, 222])
-def test_fp32c_list_is_its_gridmap_to_the_bit(ctx, field, N):
-    """The same in the precision form, with the rays its guard shot again: a
-    GridMap, its rays as a list in another order and as a served list, with 1
-    to 64 rays a bundle."""
+@pytest.mark.parametrize("N", [2, 8, 32, 33, 64, 126, 127, 128, 222])
+def test_fp32c_list_is_a_gridmap_to_the_bit(ctx, field, N):
+    """The precision form: a GridMap's rays as a list in another order and as a
+    served list.  Up to 16,000 rays they are shot in FP64, so they are the FP64
+    GridMap's results and within the form's bound of the FP32C GridMap's; beyond,
+    they are the FP32C GridMap's with the rays its guard shot again."""
     lens, _ = field
     rg = W.grid_range(300.0)
-    g = S.GridMap(lens, N, (0.0, 0.0), rg, S.SLSIM_FP32C)
-    x, n = g.positions(), N * N
+    n = N * N
+    g = S.GridMap(lens, N, (0.0, 0.0), rg, S.SLSIM_FP64 if n <= LIMIT32 else S.SLSIM_FP32C)
+    x = g.positions()
     perm = np.random.default_rng(N).permutation(n)
     y, A = g.y()[perm], g.A()[perm]
     st = {}
     assert _same(lens.rayshooterInternal(x[perm], precision=S.SLSIM_FP32C, stats=st), y, A)
-    assert st["n_guarded"] == g.stats["n_guarded"]
     srv = S.Server(ctx, hbm_budget=1 << 30)
     r = srv.wait_rays(srv.submit_rays(lens, x[perm], precision=S.SLSIM_FP32C), n)
     srv.close()
     assert _same(r, y, A)
+    g32 = S.GridMap(lens, N, (0.0, 0.0), rg, S.SLSIM_FP32C)
+    if n > LIMIT32:
+        assert st["n_guarded"] == g32.stats["n_guarded"]
+    else:
+        a = np.linalg.norm(x - g.y(), axis=1)
+        scale = np.maximum(a, 1e-3 * np.sqrt(np.mean(a ** 2)))
+        assert st["n_guarded"] == 0
+        assert (np.linalg.norm(g32.y() - g.y(), axis=1) <= 1e-5 * scale).all()
 
 
 def test_server_counts_the_rays_of_its_lists(ctx, field):
@@ -166,10 +178,10 @@ def test_server_counts_the_rays_of_its_lists(ctx, field):
 def test_rectangular_grid_is_the_grid_to_the_bit(field, N, precision):
     """A rectangular GridMap's points go as a list.  Over a power of two of
     radians with 2^k + 1 points a side they are the square GridMap's to the bit,
-    and so are its results."""
+    and so are its results (FP32C up to 16,000 rays: the FP64 one's)."""
     lens, _ = field
     rg = 2.0 ** -10
     a = S.GridMap.rect(lens, N, (0.0, 0.0), rg, rg, precision)
-    b = S.GridMap(lens, N, (0.0, 0.0), rg, precision)
+    b = S.GridMap(lens, N, (0.0, 0.0), rg, S.SLSIM_FP64 if N * N <= LIMIT32 else precision)
     assert np.array_equal(a.positions(), b.positions())
     assert _same((a.y(), a.A()), b.y(), b.A())
