@@ -43,7 +43,9 @@ enum {
                                  test within the FP32 ray's error bound of its
                                  threshold, on a cell whose flip matters) and
                                  rays with |alpha| below 1% of the call's rms
-                                 are shot again in FP64                           */
+                                 are shot again in FP64; ray lists of up to
+                                 16,000 rays through particle planes are shot in
+                                 FP64 altogether                                  */
   SLSIM_DIRECT64 = 2          /* FP64 direct sum over every particle of a plane, no
                                  tree: the error-column oracle (O(N) per ray)      */
 };
